@@ -479,6 +479,25 @@ int sgw_sigma_prod(int32_t n, int32_t n_p, int32_t num_g, const int32_t *d_nl, i
                    const sgw_complex *d_green, sgw_complex *d_array, sgw_complex *d_sigma,
                    int64_t ld_sigma, void *stream);
 
+/* The frequency loops of sigma_correlation (sigma.f90:705-745) on one W:
+ * for every term t < nterm, W continued to h_freq[t] (as sgw_analytic_eval,
+ * :714), its sigma_prod with the G(r, r') (nr, nr_p) that starts h_green[t]
+ * elements into d_green and with h_alpha[t] (:725), added to slice h_sigma[t] of d_sigma (num_g,
+ * num_g_p; leading dimension num_g; :741).  The same numbers as one
+ * sgw_analytic_eval and one sgw_sigma_prod per term, without the zero-filled
+ * nr x nr_p matrix between them.  d_work: device workspace of
+ * sgw_sigma_correlation_workspace bytes, NULL to allocate it in the call.
+ * Synchronises. */
+int64_t sgw_sigma_correlation_workspace(int32_t n, int32_t n_p, int32_t num_g, int32_t num_g_p);
+int sgw_sigma_correlation(int32_t model, int32_t num_gc, int32_t nfreq, const sgw_complex *h_z,
+                          const sgw_complex *d_coeff, int32_t nterm, const sgw_complex *h_freq,
+                          const sgw_complex *h_alpha, const int64_t *h_green,
+                          const int32_t *h_sigma, int32_t n, int32_t n_p, int32_t num_g,
+                          const int32_t *d_nl, int32_t num_g_p, const int32_t *d_nl_p,
+                          double omega, const int32_t *d_gmap, const int32_t *d_gmap_p,
+                          const sgw_complex *d_green, sgw_complex *d_sigma, void *d_work,
+                          int64_t work_bytes, void *stream);
+
 /* ---------------------------------------------------------------------------
  * Sigma_c frequency convolution (phys/corr/src/sigma.f90:705-745, the
  * accumulation sigma(:,:,isigma) += alpha * w * [G (x) W] over the Green's

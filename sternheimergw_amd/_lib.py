@@ -140,6 +140,12 @@ SIGNATURES = [
                                     c_void_p, c_void_p]),
     ("sgw_sigma_prod", c_int32, [c_int32, c_int32, c_int32, c_void_p, c_int32, c_void_p, c_double,
                                  sgw_complex, c_void_p, c_void_p, c_void_p, c_int64, c_void_p]),
+    ("sgw_sigma_correlation_workspace", c_int64, [c_int32, c_int32, c_int32, c_int32]),
+    ("sgw_sigma_correlation", c_int32, [c_int32, c_int32, c_int32, c_void_p, c_void_p, c_int32,
+                                        c_void_p, c_void_p, c_void_p, c_void_p, c_int32, c_int32,
+                                        c_int32, c_void_p, c_int32, c_void_p, c_double, c_void_p,
+                                        c_void_p, c_void_p, c_void_p, c_void_p, c_int64,
+                                        c_void_p]),
     ("sgw_broyden_create", c_void_p, [c_int64, c_int32]),
     ("sgw_broyden_destroy", None, [c_void_p]),
     ("sgw_mix_potential_c", c_int32, [c_void_p, c_int64, c_void_p, c_void_p, c_double,

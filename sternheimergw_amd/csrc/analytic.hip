@@ -406,7 +406,12 @@ __global__ void k_analytic_eval(int model, int N, Mesh m, double2 freq, int num_
   if (e >= (int64_t)num_g * num_g_p) return;
   const int r = (int)(e % num_g), c = (int)(e / num_g);
   const int64_t ne = (int64_t)num_gc * num_gc;
-  const int64_t el = (int64_t)gmap_p[c] * num_gc + gmap[r];
+  const int er = gmap[r], ec = gmap_p[c];
+  if (er < 0 || er >= num_gc || ec < 0 || ec >= num_gc) {  // no such element
+    out[(int64_t)c * nr + r] = mk(NAN, NAN);
+    return;
+  }
+  const int64_t el = (int64_t)ec * num_gc + er;
   double2 res = mk(0.0, 0.0);
   if (model == 1) {  // godby_needs_model
     const double2 c1 = coeff[el], c2 = coeff[ne + el];
@@ -477,18 +482,6 @@ __global__ void k_fill0(int64_t count, double2 *__restrict__ d) {
   if (e < count) d[e] = mk(0.0, 0.0);
 }
 
-// array(r, c) *= alpha for r < num_g, c < num_g_p; sigma(r, c) += array(r, c)
-__global__ void k_alpha_block(int num_g, int num_g_p, int64_t nr, double2 alpha,
-                              double2 *__restrict__ a, double2 *__restrict__ sigma,
-                              int64_t lds) {
-  const int64_t e = (int64_t)blockIdx.x * kEB + threadIdx.x;
-  if (e >= (int64_t)num_g * num_g_p) return;
-  const int64_t r = e % num_g, c = e / num_g;
-  const double2 v = cmul(alpha, a[c * nr + r]);
-  a[c * nr + r] = v;
-  if (sigma) sigma[c * lds + r] = cadd(sigma[c * lds + r], v);
-}
-
 template <typename F> int guarded(F &&fn) {
   try {
     return fn();
@@ -501,6 +494,46 @@ template <typename F> int guarded(F &&fn) {
   }
 }
 
+// sigma_prod of one W (block w(ldw, *)): invfft6 (sigma.f90:487), the product
+// with G(r, r') (:499) and fwfft6 (:510) into `o`.  S: num_g x nr_p scratch;
+// full: an nr x nr_p matrix, used only where the r side is not a sphere list
+// the box kernel holds.  There the first xy pass builds its planes from the
+// rows S[g][r'], the z passes of both transforms and the product are one
+// kernel, and the last xy pass keeps only the rows' positions.
+void product(hipStream_t st, const Fft6Args &a, const Fft6Lists &l, const double2 *w, int64_t ldw,
+             double2 *S, double2 *full, const double2 *green, const SphereOut &o) {
+  const int64_t nr = (int64_t)a.n * a.n * a.n, nr_p = (int64_t)a.n_p * a.n_p * a.n_p;
+  invfft6_rows(st, a, l, w, ldw, S);
+  if (l.r.fits()) {
+    SphereOut cols;
+    cols.scale = 1.0 / (double)nr;
+    cols.out = S;
+    cols.out_sg = nr_p;
+    sphere_prod(st, l.r, nr_p, -1, S, nr_p, green, cols);
+  } else {
+    // the plane lists: the G vectors of each z plane of the box
+    const int n = a.n, num_g = a.num_g;
+    std::vector<int32_t> start(n + 1, 0), gl(num_g), pos(num_g);
+    for (int g = 0; g < num_g; ++g) ++start[l.nl[g] / (n * n) + 1];
+    for (int z = 0; z < n; ++z) start[z + 1] += start[z];
+    std::vector<int32_t> fill(start.begin(), start.end() - 1);
+    for (int g = 0; g < num_g; ++g) {
+      const int k = fill[l.nl[g] / (n * n)]++;
+      gl[k] = g;
+      pos[k] = l.nl[g] % (n * n);
+    }
+    DevBuf<int32_t> d_start(n + 1), d_gl(num_g), d_pos(num_g);
+    d_start.upload(start.data(), n + 1, st);
+    d_gl.upload(gl.data(), num_g, st);
+    d_pos.upload(pos.data(), num_g, st);
+    box_xy_scatter(st, n, nr_p, S, d_start.p, d_gl.p, d_pos.p, full, -1);
+    box_z_product(st, n, nr_p, full, green);
+    box_xy_gather(st, n, nr_p, full, d_start.p, d_gl.p, d_pos.p, 1.0 / (double)nr, S, +1);
+    SGW_HIP(hipStreamSynchronize(st));  // the plane lists are freed here
+  }
+  fwfft6_rows(st, a, l, S, o);                                            // :519-521
+}
+
 Mesh make_mesh(int N, const sgw_complex *h_z, const int32_t *h_src) {
   SGW_REQUIRE(N >= 1 && N <= kMaxPade, SGW_E_SHAPE, "analytic: 1 <= frequencies <= 64");
   Mesh m{};
@@ -509,6 +542,32 @@ Mesh make_mesh(int N, const sgw_complex *h_z, const int32_t *h_src) {
     m.src[i] = h_src ? h_src[i] : i;
   }
   return m;
+}
+
+// the arguments of an evaluation; returns the mesh the model needs
+Mesh eval_check(int32_t model, int32_t num_gc, int32_t nfreq, const sgw_complex *h_z,
+                const sgw_complex *d_coeff, int32_t n, int32_t n_p, int32_t num_g,
+                int32_t num_g_p, const int32_t *d_gmap, const int32_t *d_gmap_p) {
+  (void)num_gc;
+  const bool self_contained =
+      model == SGW_PADE_ROBUST || model == SGW_AAA_APPROX || model == SGW_AAA_POLE;
+  SGW_REQUIRE(d_coeff && d_gmap && d_gmap_p && (h_z || self_contained), SGW_E_ARG,
+              "analytic_eval: null argument");
+  SGW_REQUIRE(model >= SGW_GODBY_NEEDS && model <= SGW_AAA_POLE, SGW_E_ARG,
+              "analytic_eval: model must be SGW_GODBY_NEEDS, SGW_PADE_APPROX, SGW_PADE_ROBUST, "
+              "SGW_AAA_APPROX or SGW_AAA_POLE");
+  SGW_REQUIRE(model != SGW_AAA_APPROX || (nfreq >= 3 && nfreq <= kMaxPade), SGW_E_SHAPE,
+              "analytic_eval: AAA coefficients need 3..64 slices");
+  SGW_REQUIRE(model != SGW_AAA_POLE || (nfreq >= 2 && nfreq <= kMaxPade), SGW_E_SHAPE,
+              "analytic_eval: AAA pole coefficients need 2..64 slices");
+  SGW_REQUIRE(model != SGW_PADE_ROBUST || (nfreq >= 4 && nfreq <= kMaxPade), SGW_E_SHAPE,
+              "analytic_eval: robust Pade coefficients need 4..64 slices");
+  SGW_REQUIRE(model != SGW_GODBY_NEEDS || nfreq == 2, SGW_E_SHAPE,
+              "analytic_eval: Godby-Needs uses 2 coefficients");
+  const int64_t nr = (int64_t)n * n * n, nr_p = (int64_t)n_p * n_p * n_p;
+  SGW_REQUIRE(num_g >= 1 && num_g <= nr && num_g_p >= 1 && num_g_p <= nr_p, SGW_E_SHAPE,
+              "analytic_eval: need num_g <= n^3 and num_g_p <= n_p^3");
+  return self_contained ? Mesh{} : make_mesh(nfreq, h_z, nullptr);
 }
 
 }  // namespace
@@ -574,25 +633,10 @@ extern "C" int sgw_analytic_eval(int32_t model, int32_t num_gc, int32_t nfreq,
                                  int32_t num_g_p, const int32_t *d_gmap,
                                  const int32_t *d_gmap_p, sgw_complex *d_out, void *stream) {
   return guarded([&] {
-    const bool self_contained =
-        model == SGW_PADE_ROBUST || model == SGW_AAA_APPROX || model == SGW_AAA_POLE;
-    SGW_REQUIRE(d_coeff && d_gmap && d_gmap_p && d_out && (h_z || self_contained), SGW_E_ARG,
-                "analytic_eval: null argument");
-    SGW_REQUIRE(model >= SGW_GODBY_NEEDS && model <= SGW_AAA_POLE, SGW_E_ARG,
-                "analytic_eval: model must be SGW_GODBY_NEEDS, SGW_PADE_APPROX, SGW_PADE_ROBUST, "
-                "SGW_AAA_APPROX or SGW_AAA_POLE");
-    SGW_REQUIRE(model != SGW_AAA_APPROX || (nfreq >= 3 && nfreq <= kMaxPade), SGW_E_SHAPE,
-                "analytic_eval: AAA coefficients need 3..64 slices");
-    SGW_REQUIRE(model != SGW_AAA_POLE || (nfreq >= 2 && nfreq <= kMaxPade), SGW_E_SHAPE,
-                "analytic_eval: AAA pole coefficients need 2..64 slices");
-    SGW_REQUIRE(model != SGW_PADE_ROBUST || (nfreq >= 4 && nfreq <= kMaxPade), SGW_E_SHAPE,
-                "analytic_eval: robust Pade coefficients need 4..64 slices");
-    SGW_REQUIRE(model != SGW_GODBY_NEEDS || nfreq == 2, SGW_E_SHAPE,
-                "analytic_eval: Godby-Needs uses 2 coefficients");
+    SGW_REQUIRE(d_out != nullptr, SGW_E_ARG, "analytic_eval: null argument");
+    const Mesh m = eval_check(model, num_gc, nfreq, h_z, d_coeff, n, n_p, num_g, num_g_p, d_gmap,
+                              d_gmap_p);
     const int64_t nr = (int64_t)n * n * n, nr_p = (int64_t)n_p * n_p * n_p;
-    SGW_REQUIRE(num_g >= 1 && num_g <= nr && num_g_p >= 1 && num_g_p <= nr_p, SGW_E_SHAPE,
-                "analytic_eval: need num_g <= n^3 and num_g_p <= n_p^3");
-    const Mesh m = self_contained ? Mesh{} : make_mesh(nfreq, h_z, nullptr);
     hipStream_t st = (hipStream_t)stream;
     double2 *out = reinterpret_cast<double2 *>(d_out);
     KScope ks("analytic_eval", st);
@@ -617,41 +661,81 @@ extern "C" int sgw_sigma_prod(int32_t n, int32_t n_p, int32_t num_g, const int32
     fft6_check(a, "sigma_prod");
     hipStream_t st = (hipStream_t)stream;
     const int64_t nr = (int64_t)n * n * n, nr_p = (int64_t)n_p * n_p * n_p;
+    const Fft6Lists lists(st, a, "sigma_prod");
     DevBuf<double2> S((size_t)num_g * nr_p);
-    KScope ks("sigma_prod", st);
-    // invfft6 (sigma.f90:487), the product with G (:499) and fwfft6 (:510).
-    // Along r: the first xy pass builds its planes from the rows S[g][r']
-    // (no zero-filled matrix in HBM), the z passes of both transforms and
-    // the product are one kernel, and the last xy pass keeps only the rows'
-    // positions.  The plane lists: the G vectors of each z plane of the box.
-    std::vector<int32_t> nl(num_g);
-    SGW_HIP(hipMemcpyAsync(nl.data(), d_nl, sizeof(int32_t) * num_g, hipMemcpyDeviceToHost, st));
-    SGW_HIP(hipStreamSynchronize(st));
-    for (int g = 0; g < num_g; ++g)
-      SGW_REQUIRE(nl[g] >= 0 && nl[g] < nr, SGW_E_ARG, "sigma_prod: box index out of range");
-    std::vector<int32_t> start(n + 1, 0), gl(num_g), pos(num_g);
-    for (int g = 0; g < num_g; ++g) ++start[nl[g] / (n * n) + 1];
-    for (int z = 0; z < n; ++z) start[z + 1] += start[z];
-    std::vector<int32_t> fill(start.begin(), start.end() - 1);
-    for (int g = 0; g < num_g; ++g) {
-      const int k = fill[nl[g] / (n * n)]++;
-      gl[k] = g;
-      pos[k] = nl[g] % (n * n);
+    {
+      KScope ks("sigma_prod", st);
+      SphereOut o;
+      o.has_alpha = true;
+      o.alpha = make_double2(alpha.re, alpha.im);
+      o.out = a.f;
+      o.out_sg = nr;
+      o.sum = reinterpret_cast<double2 *>(d_sigma);                       // :741
+      o.sum_sg = ld_sigma;
+      product(st, a, lists, a.f, nr, S.p, a.f, reinterpret_cast<const double2 *>(d_green), o);
     }
-    DevBuf<int32_t> d_start(n + 1), d_gl(num_g), d_pos(num_g);
-    d_start.upload(start.data(), n + 1, st);
-    d_gl.upload(gl.data(), num_g, st);
-    d_pos.upload(pos.data(), num_g, st);
-    invfft6_rows(st, a, S.p, 0);
-    box_xy_scatter(st, n, nr_p, S.p, d_start.p, d_gl.p, d_pos.p, a.f, -1);
-    box_z_product(st, n, nr_p, a.f, reinterpret_cast<const double2 *>(d_green));
-    box_xy_gather(st, n, nr_p, a.f, d_start.p, d_gl.p, d_pos.p, 1.0 / (double)nr, S.p, +1);
-    fwfft6_rows(st, a, S.p, 0);
-    k_alpha_block<<<blocks((int64_t)num_g * num_g_p), kEB, 0, st>>>(
-        num_g, num_g_p, nr, make_double2(alpha.re, alpha.im), a.f,
-        reinterpret_cast<double2 *>(d_sigma), ld_sigma);                  // :519-521, :741
     SGW_HIP(hipGetLastError());
     SGW_HIP(hipStreamSynchronize(st));  // scratch freed on return
+    return 0;
+  });
+}
+
+extern "C" int64_t sgw_sigma_correlation_workspace(int32_t n, int32_t n_p, int32_t num_g,
+                                                   int32_t num_g_p) {
+  if (n < 1 || n_p < 1 || num_g < 1 || num_g_p < 1) return 0;
+  const int64_t nr_p = (int64_t)n_p * n_p * n_p;
+  return (int64_t)sizeof(double2) * ((int64_t)num_g * nr_p + (int64_t)num_g * num_g_p);
+}
+
+extern "C" int sgw_sigma_correlation(
+    int32_t model, int32_t num_gc, int32_t nfreq, const sgw_complex *h_z,
+    const sgw_complex *d_coeff, int32_t nterm, const sgw_complex *h_freq,
+    const sgw_complex *h_alpha, const int64_t *h_green, const int32_t *h_sigma, int32_t n,
+    int32_t n_p, int32_t num_g, const int32_t *d_nl, int32_t num_g_p, const int32_t *d_nl_p,
+    double omega, const int32_t *d_gmap, const int32_t *d_gmap_p, const sgw_complex *d_green,
+    sgw_complex *d_sigma, void *d_work, int64_t work_bytes, void *stream) {
+  return guarded([&] {
+    const Mesh m = eval_check(model, num_gc, nfreq, h_z, d_coeff, n, n_p, num_g, num_g_p, d_gmap,
+                              d_gmap_p);
+    SGW_REQUIRE(nterm >= 0 && (nterm == 0 || (h_freq && h_alpha && h_green && h_sigma)) &&
+                    d_green && d_sigma,
+                SGW_E_ARG, "sigma_correlation: null argument or negative count");
+    const int64_t need = sgw_sigma_correlation_workspace(n, n_p, num_g, num_g_p);
+    SGW_REQUIRE(!d_work || work_bytes >= need, SGW_E_SHAPE,
+                "sigma_correlation: workspace too small");
+    // the check's matrix pointer; the box kernels need no full matrix
+    Fft6Args a{n, n_p, num_g, num_g_p, d_nl, d_nl_p, omega, 1,
+               reinterpret_cast<double2 *>(d_sigma)};
+    fft6_check(a, "sigma_correlation");
+    for (int t = 0; t < nterm; ++t)
+      SGW_REQUIRE(h_green[t] >= 0 && h_sigma[t] >= 0, SGW_E_ARG,
+                  "sigma_correlation: negative slice");
+    hipStream_t st = (hipStream_t)stream;
+    const int64_t nr = (int64_t)n * n * n, nr_p = (int64_t)n_p * n_p * n_p;
+    const Fft6Lists lists(st, a, "sigma_correlation");
+    DevBuf<double2> own, full;
+    if (!d_work) own.alloc((size_t)need / sizeof(double2));
+    if (!lists.r.fits()) full.alloc((size_t)(nr * nr_p));
+    double2 *S = d_work ? static_cast<double2 *>(d_work) : own.p, *W = S + num_g * nr_p;
+    for (int t = 0; t < nterm; ++t) {
+      {
+        KScope ks("analytic_eval", st);
+        k_analytic_eval<<<blocks((int64_t)num_g * num_g_p), kEB, 0, st>>>(
+            model, nfreq, m, make_double2(h_freq[t].re, h_freq[t].im), num_gc,
+            reinterpret_cast<const double2 *>(d_coeff), num_g, num_g_p, d_gmap, d_gmap_p, num_g,
+            W);
+      }
+      KScope ks("sigma_prod", st);
+      SphereOut o;
+      o.has_alpha = true;
+      o.alpha = make_double2(h_alpha[t].re, h_alpha[t].im);
+      o.sum = reinterpret_cast<double2 *>(d_sigma) + (int64_t)h_sigma[t] * num_g * num_g_p;
+      o.sum_sg = num_g;
+      product(st, a, lists, W, num_g, S, full.p,
+              reinterpret_cast<const double2 *>(d_green) + h_green[t], o);
+    }
+    SGW_HIP(hipGetLastError());
+    SGW_HIP(hipStreamSynchronize(st));  // the lists are freed on return
     return 0;
   });
 }

@@ -212,17 +212,6 @@ void box_fft(hipStream_t st, int n, int64_t nvec, double2 *d, int sign) {
     dispatch<-1>(st, n, nvec, d);
 }
 
-void box_fft_xy(hipStream_t st, int n, int64_t nvec, double2 *d, int sign) {
-  if (nvec <= 0) return;
-  with_side(n, [&](auto side) {
-    constexpr int N = decltype(side)::value;
-    if (sign > 0)
-      k_box_xy<N, 1><<<(unsigned)(nvec * N), 64, 0, st>>>(d);
-    else
-      k_box_xy<N, -1><<<(unsigned)(nvec * N), 64, 0, st>>>(d);
-  });
-}
-
 void box_xy_scatter(hipStream_t st, int n, int64_t nvec, const double2 *S, const int32_t *start,
                     const int32_t *gl, const int32_t *pos, double2 *d, int sign) {
   if (nvec <= 0) return;

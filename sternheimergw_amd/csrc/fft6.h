@@ -3,6 +3,7 @@
 #pragma once
 
 #include "sgw_internal.h"
+#include "spherefft.h"
 
 namespace sgw {
 
@@ -16,16 +17,21 @@ struct Fft6Args {
 
 void fft6_check(const Fft6Args &a, const char *who);
 
-// One matrix at a time on `st`; `scratch` holds num_g * n_p^3 elements.
-void invfft6_run(hipStream_t st, const Fft6Args &a, double2 *scratch);
-void fwfft6_run(hipStream_t st, const Fft6Args &a, double2 *scratch);
-// The parts of matrix m: invfft6 = front, then box_fft(n, n_p^3, f_m, -1);
-// fwfft6 = box_fft(n, n_p^3, f_m, +1), then back.
-void invfft6_front(hipStream_t st, const Fft6Args &a, double2 *scratch, int m);
-void fwfft6_back(hipStream_t st, const Fft6Args &a, double2 *scratch, int m);
-// The r' sides alone: invfft6_front = invfft6_rows, then the zero-filled
-// box scatter of the rows; fwfft6_back = the box gather, then fwfft6_rows.
-void invfft6_rows(hipStream_t st, const Fft6Args &a, double2 *scratch, int m);
-void fwfft6_rows(hipStream_t st, const Fft6Args &a, double2 *scratch, int m);
+// The two G lists on the host and, where the box kernels of spherefft.h take
+// them, as sphere lists on the device.  Reads the maps back from the device
+// (synchronises `st`) and rejects indices outside the boxes.
+struct Fft6Lists {
+  Fft6Lists(hipStream_t st, const Fft6Args &a, const char *who);
+  std::vector<int32_t> nl, nl_p;
+  SphereList r, r_p;
+};
+
+// Scratch of one matrix: S[g][r'] (num_g x n_p^3).  One matrix at a time on
+// `st`; the parts below work on matrix f(ldf, *) with its block at the top
+// left.  rows: the r' side, S[g] = box FFT of the rows of f, and back.
+void invfft6_rows(hipStream_t st, const Fft6Args &a, const Fft6Lists &l, const double2 *f,
+                  int64_t ldf, double2 *s);
+void fwfft6_rows(hipStream_t st, const Fft6Args &a, const Fft6Lists &l, double2 *s,
+                 SphereOut out);
 
 }  // namespace sgw

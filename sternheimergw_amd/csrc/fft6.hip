@@ -11,15 +11,20 @@
 //   fwfft6:  f(G, G') = Omega / (nr nr_p) sum_{r,r'} e^{+iGr} f(r, r') e^{-iG'r'}
 // The reference gets the e^{-iGr} of the first index by conjugating around
 // QE's invfft / fwfft (fft6.f90:148-162, 323-338); here the box FFT runs
-// with the opposite sign directly.  Each transform is two batched box-FFT
-// passes with one scratch matrix S[g][r'] (num_g x nr_p) between them:
+// with the opposite sign directly.  Each transform is two batched steps with
+// one scratch matrix S[g][r'] (num_g x nr_p) between them:
 //   invfft6: S[g] = invfft_p(scatter_p(f(g, :) / Omega))     (rows)
 //            f(:, r') = fft_(-)(scatter(S[:, r']))            (columns, in place)
 //   fwfft6:  f(:, r') = fft_(+)(f(:, r'))                      (columns, in place)
 //            S[g][r'] = f(nl[g], r') / nr
 //            f(g, g') = Omega / nr_p fft_(-)(S[g])(nl_p[g'])  (rows)
-// Index-map kernels put the contiguous index of both operands on adjacent
-// lanes where one side is a gather.
+// A step is one kernel of spherefft.h, which keeps each box in LDS and
+// registers and reads the list values and the real-space side once (a call of
+// invfft6 with 1536 x 455 G on 24^3 x 16^3: 635 us against 1531 through the
+// passes; 455 x 455 on 16^3: 177 against 366, fwfft6 171 against 282).  Sides and lists it does not hold run as
+// index-map kernels around whole-box FFT passes, as below; those put the
+// contiguous index of both operands on adjacent lanes where one side is a
+// gather.
 #include <algorithm>
 
 #include "boxfft.h"
@@ -69,15 +74,21 @@ __global__ void k_cols_gather(int num_g, int64_t nr, int64_t nr_p, const int32_t
   S[e] = mk(s * v.x, s * v.y);
 }
 
-// f[j * nr + g] = s * S[g][nl_p[j]]
-__global__ void k_rows_gather(int num_g, int num_g_p, int64_t nr, int64_t nr_p,
+// v = o.scale * S[g][nl_p[j]], times o.alpha, to o.out[j][g] and into o.sum[j][g]
+__global__ void k_rows_gather(int num_g, int num_g_p, int64_t nr_p,
                               const int32_t *__restrict__ nl_p, const double2 *__restrict__ S,
-                              double s, double2 *__restrict__ f) {
+                              SphereOut o) {
   const int64_t e = (int64_t)blockIdx.x * kEB + threadIdx.x;
   if (e >= (int64_t)num_g * num_g_p) return;
   const int64_t g = e % num_g, j = e / num_g;
-  const double2 v = S[g * nr_p + nl_p[j]];
-  f[j * nr + g] = mk(s * v.x, s * v.y);
+  const double2 t = S[g * nr_p + nl_p[j]];
+  double2 v = mk(o.scale * t.x, o.scale * t.y);
+  if (o.has_alpha) v = cmul(o.alpha, v);
+  if (o.out) o.out[j * o.out_sg + g] = v;
+  if (o.sum) {
+    double2 *p = o.sum + j * o.sum_sg + g;
+    *p = cadd(*p, v);
+  }
 }
 
 // green[f][c][r] = x[colsys[c]][f][rowmap[r]] where both maps are >= 0 and
@@ -123,61 +134,90 @@ void fft6_check(const Fft6Args &a, const char *who) {
   SGW_REQUIRE(a.omega > 0.0, SGW_E_ARG, std::string(who) + ": the cell volume must be positive");
 }
 
-// invfft6 of matrix m, r' side only: S[g][r'] for the num_g rows
-void invfft6_rows(hipStream_t st, const Fft6Args &a, double2 *s, int m) {
-  const int n = a.n, n_p = a.n_p, num_g = a.num_g, num_g_p = a.num_g_p;
-  const int64_t nr = (int64_t)n * n * n, nr_p = (int64_t)n_p * n_p * n_p;
-  double2 *f = a.f + (int64_t)m * nr * nr_p;
+Fft6Lists::Fft6Lists(hipStream_t st, const Fft6Args &a, const char *who)
+    : nl(a.num_g), nl_p(a.num_g_p) {
+  SGW_HIP(hipMemcpyAsync(nl.data(), a.nl, sizeof(int32_t) * a.num_g, hipMemcpyDeviceToHost, st));
+  SGW_HIP(hipMemcpyAsync(nl_p.data(), a.nl_p, sizeof(int32_t) * a.num_g_p, hipMemcpyDeviceToHost,
+                         st));
+  SGW_HIP(hipStreamSynchronize(st));
+  const int nr = a.n * a.n * a.n, nr_p = a.n_p * a.n_p * a.n_p;
+  for (int32_t p : nl)
+    SGW_REQUIRE(p >= 0 && p < nr, SGW_E_ARG, std::string(who) + ": box index out of range");
+  for (int32_t p : nl_p)
+    SGW_REQUIRE(p >= 0 && p < nr_p, SGW_E_ARG, std::string(who) + ": box index out of range");
+  r = SphereList(a.n, nl);
+  r_p = SphereList(a.n_p, nl_p);
+  r.upload(st);
+  r_p.upload(st);
+}
+
+void invfft6_rows(hipStream_t st, const Fft6Args &a, const Fft6Lists &l, const double2 *f,
+                  int64_t ldf, double2 *s) {
+  const int num_g = a.num_g, num_g_p = a.num_g_p;
+  const int64_t nr_p = (int64_t)a.n_p * a.n_p * a.n_p;
+  if (l.r_p.fits()) {
+    sphere_inv(st, l.r_p, num_g, +1, f, ldf, 1.0 / a.omega, s);
+    return;
+  }
   k_fill0<<<blocks((int64_t)num_g * nr_p), kEB, 0, st>>>((int64_t)num_g * nr_p, s);
-  k_rows_scatter<<<blocks((int64_t)num_g * num_g_p), kEB, 0, st>>>(
-      num_g, num_g_p, nr, nr_p, a.nl_p, f, 1.0 / a.omega, s);
-  box_fft(st, n_p, num_g, s, +1);
+  k_rows_scatter<<<blocks((int64_t)num_g * num_g_p), kEB, 0, st>>>(num_g, num_g_p, ldf, nr_p,
+                                                                    a.nl_p, f, 1.0 / a.omega, s);
+  box_fft(st, a.n_p, num_g, s, +1);
 }
 
-// fwfft6 of matrix m, r' side only, from S[g][r'] into the block of f
-void fwfft6_rows(hipStream_t st, const Fft6Args &a, double2 *s, int m) {
-  const int n = a.n, n_p = a.n_p, num_g = a.num_g, num_g_p = a.num_g_p;
-  const int64_t nr = (int64_t)n * n * n, nr_p = (int64_t)n_p * n_p * n_p;
-  double2 *f = a.f + (int64_t)m * nr * nr_p;
-  box_fft(st, n_p, num_g, s, -1);
-  k_rows_gather<<<blocks((int64_t)num_g * num_g_p), kEB, 0, st>>>(
-      num_g, num_g_p, nr, nr_p, a.nl_p, s, a.omega / (double)nr_p, f);
+void fwfft6_rows(hipStream_t st, const Fft6Args &a, const Fft6Lists &l, double2 *s,
+                 SphereOut o) {
+  const int64_t nr_p = (int64_t)a.n_p * a.n_p * a.n_p;
+  o.scale = a.omega / (double)nr_p;
+  if (l.r_p.fits()) {
+    sphere_fwd(st, l.r_p, a.num_g, -1, s, o);
+    return;
+  }
+  box_fft(st, a.n_p, a.num_g, s, -1);
+  k_rows_gather<<<blocks((int64_t)a.num_g * a.num_g_p), kEB, 0, st>>>(a.num_g, a.num_g_p, nr_p,
+                                                                     a.nl_p, s, o);
 }
 
-// invfft6 of matrix m up to its last pass: f(r, r') in G along r, r' in r'
-// space; the r transform is left to the caller
-void invfft6_front(hipStream_t st, const Fft6Args &a, double2 *s, int m) {
-  const int64_t nr = (int64_t)a.n * a.n * a.n, nr_p = (int64_t)a.n_p * a.n_p * a.n_p;
-  double2 *f = a.f + (int64_t)m * nr * nr_p;
-  invfft6_rows(st, a, s, m);
-  k_fill0<<<blocks(nr * nr_p), kEB, 0, st>>>(nr * nr_p, f);
-  k_cols_scatter<<<blocks((int64_t)a.num_g * nr_p), kEB, 0, st>>>(a.num_g, nr, nr_p, a.nl, s, f);
-}
+namespace {
 
-// fwfft6 of matrix m from after its first pass (f already transformed along r)
-void fwfft6_back(hipStream_t st, const Fft6Args &a, double2 *s, int m) {
-  const int64_t nr = (int64_t)a.n * a.n * a.n, nr_p = (int64_t)a.n_p * a.n_p * a.n_p;
-  double2 *f = a.f + (int64_t)m * nr * nr_p;
-  k_cols_gather<<<blocks((int64_t)a.num_g * nr_p), kEB, 0, st>>>(a.num_g, nr, nr_p, a.nl, f,
-                                                                  1.0 / (double)nr, s);
-  fwfft6_rows(st, a, s, m);
-}
-
-void invfft6_run(hipStream_t st, const Fft6Args &a, double2 *s) {
+void invfft6_run(hipStream_t st, const Fft6Args &a, const Fft6Lists &l, double2 *s) {
   const int64_t nr = (int64_t)a.n * a.n * a.n, nr_p = (int64_t)a.n_p * a.n_p * a.n_p;
   for (int m = 0; m < a.nmat; ++m) {
-    invfft6_front(st, a, s, m);
-    box_fft(st, a.n, nr_p, a.f + (int64_t)m * nr * nr_p, -1);
+    double2 *f = a.f + (int64_t)m * nr * nr_p;
+    invfft6_rows(st, a, l, f, nr, s);
+    if (l.r.fits()) {
+      sphere_inv(st, l.r, nr_p, -1, s, nr_p, 1.0, f);
+      continue;
+    }
+    k_fill0<<<blocks(nr * nr_p), kEB, 0, st>>>(nr * nr_p, f);
+    k_cols_scatter<<<blocks((int64_t)a.num_g * nr_p), kEB, 0, st>>>(a.num_g, nr, nr_p, a.nl, s, f);
+    box_fft(st, a.n, nr_p, f, -1);
   }
 }
 
-void fwfft6_run(hipStream_t st, const Fft6Args &a, double2 *s) {
+void fwfft6_run(hipStream_t st, const Fft6Args &a, const Fft6Lists &l, double2 *s) {
   const int64_t nr = (int64_t)a.n * a.n * a.n, nr_p = (int64_t)a.n_p * a.n_p * a.n_p;
   for (int m = 0; m < a.nmat; ++m) {
-    box_fft(st, a.n, nr_p, a.f + (int64_t)m * nr * nr_p, +1);
-    fwfft6_back(st, a, s, m);
+    double2 *f = a.f + (int64_t)m * nr * nr_p;
+    SphereOut rows;
+    if (l.r.fits()) {
+      SphereOut cols;
+      cols.scale = 1.0 / (double)nr;
+      cols.out = s;
+      cols.out_sg = nr_p;
+      sphere_fwd(st, l.r, nr_p, +1, f, cols);
+    } else {
+      box_fft(st, a.n, nr_p, f, +1);
+      k_cols_gather<<<blocks((int64_t)a.num_g * nr_p), kEB, 0, st>>>(a.num_g, nr, nr_p, a.nl, f,
+                                                                      1.0 / (double)nr, s);
+    }
+    rows.out = f;
+    rows.out_sg = nr;
+    fwfft6_rows(st, a, l, s, rows);
   }
 }
+
+}  // namespace
 
 }  // namespace sgw
 
@@ -191,9 +231,10 @@ extern "C" int sgw_invfft6(int32_t n, int32_t n_p, int32_t num_g, const int32_t 
                reinterpret_cast<double2 *>(d_f)};
     fft6_check(a, "invfft6");
     hipStream_t st = (hipStream_t)stream;
+    const Fft6Lists lists(st, a, "invfft6");
     DevBuf<double2> S((size_t)num_g * n_p * n_p * n_p);  // one matrix at a time
     KScope ks("invfft6", st);
-    invfft6_run(st, a, S.p);
+    invfft6_run(st, a, lists, S.p);
     SGW_HIP(hipGetLastError());
     SGW_HIP(hipStreamSynchronize(st));  // scratch freed on return
     return 0;
@@ -208,9 +249,10 @@ extern "C" int sgw_fwfft6(int32_t n, int32_t n_p, int32_t num_g, const int32_t *
                reinterpret_cast<double2 *>(d_f)};
     fft6_check(a, "fwfft6");
     hipStream_t st = (hipStream_t)stream;
+    const Fft6Lists lists(st, a, "fwfft6");
     DevBuf<double2> S((size_t)num_g * n_p * n_p * n_p);
     KScope ks("fwfft6", st);
-    fwfft6_run(st, a, S.p);
+    fwfft6_run(st, a, lists, S.p);
     SGW_HIP(hipGetLastError());
     SGW_HIP(hipStreamSynchronize(st));
     return 0;

@@ -123,14 +123,24 @@ def sigma_correlation(grid: CorrGrid, grid_p: CorrGrid, omega_cell: float, alpha
     d_gm, d_gmp = torch.from_numpy(gm).to(dev), torch.from_numpy(gmp).to(dev)
     sigma = torch.zeros((freq_sigma.size, grid_p.num_g, grid.num_g), dtype=torch.complex128,
                         device=dev)
-    work = torch.empty((grid_p.nr, grid.nr), dtype=torch.complex128, device=dev)
-    for isig, fs in enumerate(freq_sigma):
-        for ig, fg in enumerate(freq_green):
-            fc = fs - fg                                             # sigma.f90:709
-            if fc.real * fc.imag < 0.0:                              # :711
-                fc = np.conj(fc)
-            w.eval_into(fc, grid, grid_p, d_gm, d_gmp, work)         # :714
-            icoul = ig % num_coul                                    # :722
-            sigma_prod(grid, grid_p, omega_cell, alpha * weight[icoul], d_green_r[ig], work,
-                       sigma[isig])                                  # :725, :741
+    nterm = freq_sigma.size * freq_green.size
+    freq = np.empty(nterm, dtype=np.complex128)
+    alphas = np.empty(nterm, dtype=np.complex128)
+    igs = np.tile(np.arange(freq_green.size, dtype=np.int32), freq_sigma.size)
+    isig = np.repeat(np.arange(freq_sigma.size, dtype=np.int32), freq_green.size)
+    for t in range(nterm):
+        fc = freq_sigma[isig[t]] - freq_green[igs[t]]                # sigma.f90:709
+        if fc.real * fc.imag < 0.0:                                  # :711
+            fc = np.conj(fc)
+        freq[t] = w.symmetrize(fc)                                   # :714
+        alphas[t] = alpha * weight[igs[t] % num_coul]                # :722, :725
+    at = igs.astype(np.int64) * d_green_r.stride(0)
+    lib = _lib.lib()
+    need = lib.sgw_sigma_correlation_workspace(grid.n, grid_p.n, grid.num_g, grid_p.num_g)
+    work = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
+    _lib.check(lib.sgw_sigma_correlation(
+        w.model, w.num_g, w.z.size, w._hz, _p(w.coeff), nterm, _lib.ptr(freq), _lib.ptr(alphas),
+        _lib.ptr(at), _lib.ptr(isig), grid.n, grid_p.n, grid.num_g, _p(grid.d_nl), grid_p.num_g,
+        _p(grid_p.d_nl), omega_cell, _p(d_gm), _p(d_gmp), _p(d_green_r), _p(sigma), _p(work),
+        need, _stream()))
     return sigma
