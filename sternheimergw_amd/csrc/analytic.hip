@@ -3,7 +3,7 @@
 //    the Godby-Needs plasmon-pole model (godby_needs.f90) and the N-point
 //    Pade approximant of Vidberg and Serene (pade.f90:41-147), one thread per
 //    (G, G') element, and the robust Pade approximant (pade_robust.f90), one
-//    group of 32 lanes per element;
+//    group of 16 or 32 lanes per element;
 //  * sigma_prod (phys/corr/src/sigma.f90:417-523): W(G, G') -> W(r, r') by
 //    invfft6, the product G(r, r') W(r, r'), fwfft6 back, times alpha, and
 //    optionally added into Sigma (sigma.f90:741).
@@ -15,6 +15,7 @@
 #include "boxfft.h"
 #include "fft6.h"
 #include "ktimer.h"
+#include "lanes.h"
 #include "sgw_internal.h"
 
 namespace sgw {
@@ -93,130 +94,224 @@ __global__ void k_pade_coeffs(int64_t ne, int N, Mesh m, double2 *__restrict__ w
 // ---------------------------------------------------------------------------
 // Robust Pade approximation (pade_robust.f90:164-535, the SVD algorithm of
 // P. Gonnet, S. Guettel and L. N. Trefethen, SIAM Rev. 55 (2013) 101-117)
-// of every element from its values on a circle of N points.  One group of 32
-// lanes (half a wavefront) per element; lane l holds row l of the group's
-// matrix, which lives in LDS column by column (column stride 32).  Numerical
-// rank from one-sided Jacobi singular values (the reference calls ZGESDD);
-// null vectors from Householder QR in the form of ZGEQRF + ZUNGQR (the
-// reference's qr wrapper, lapack.f90:150-225).
+// of every element from its values on a circle of N points.  One group of G
+// lanes per element; lane l holds row l of the group's matrix, which lives in
+// LDS column by column (column stride G).  The matrices have at most
+// N/2 - 1 rows, so up to 35 points a quarter wavefront (G = 16) carries an
+// element, above that half a wavefront; the group reductions give the same
+// bits either way.  Numerical rank from one-sided Jacobi singular values (the
+// reference calls ZGESDD); null vectors from Householder QR in the form of
+// ZGEQRF + ZUNGQR (the reference's qr wrapper, lapack.f90:150-225).
+//
+// Bound: the chains of dependent FP64 instructions of the Jacobi pairs (HBM
+// moves 2 x 16 N bytes per element).  400 x 400 elements of six poles, N = 32:
+// 52.4 ms with half a wavefront per element, LDS-permute sums and full Jacobi;
+// 14.5 ms with vector sums, quarter wavefronts and Jacobi left once the rank
+// is certain; 12.1 ms with a pair's columns kept in registers; 2.4 ms with the
+// pivoted QR deciding first (96 % of these elements; the other 4 % take half
+// of the time that is left).
 
-constexpr int kPrLanes = 32;                            // lanes per element
-constexpr int kPrGroups = 4;                            // most elements per block
+constexpr int kPrBlock = 128;                           // most threads per block
 constexpr int kPrLdsMax = 65536;                        // LDS bytes per block
 constexpr int kPrSweeps = 40;                           // Jacobi sweep limit
 constexpr double kPrTol = 1e-14;                        // eps14, the default tolerance
 constexpr double kSqrtEps = 1.4901161193847656e-08;     // sqrt(epsilon(1.0_dp))
 constexpr double kDblEps = 2.220446049250313e-16;
+constexpr int kPrSmallMax = 35;                         // most points with G = 16
 
-// LDS per element: f then a (64), Taylor coefficients (64), b (32), tau (32),
-// the matrix (32 x nmax)
-__host__ __device__ inline int pr_group_lds(int nmax) { return 192 + kPrLanes * nmax; }
+// LDS per element: Taylor coefficients (2 G), b (G), tau (G), the matrix
+// (G x nmax), whose place the samples take before it and a after it (at least
+// N: nmax = N / 2 - 2 >= 3)
+template <int G> __host__ __device__ inline int pr_group_lds(int nmax) {
+  return 4 * G + G * nmax;
+}
 
-// sums and extrema over the 32 lanes of a group; the butterfly gives every
-// lane the same bits (each stage adds the same two operands)
-__device__ inline double gsum(double v) {
-#pragma unroll
-  for (int o = kPrLanes / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, kPrLanes);
-  return v;
-}
-__device__ inline double gmax(double v) {
-#pragma unroll
-  for (int o = kPrLanes / 2; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, kPrLanes));
-  return v;
-}
-__device__ inline int gmaxi(int v) {
-#pragma unroll
-  for (int o = kPrLanes / 2; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, kPrLanes));
-  return v;
-}
-__device__ inline int gmini(int v) {
-#pragma unroll
-  for (int o = kPrLanes / 2; o > 0; o >>= 1) v = min(v, __shfl_xor(v, o, kPrLanes));
-  return v;
-}
 __device__ inline double cabsd(double2 a) { return hypot(a.x, a.y); }
 
 // row l of (C D)^T: A(l, i) = C(i, l) d_l = c(m+1+i-l) d_l for i < n, l <= n,
 // C = rows m+1..m+n of the Toeplitz matrix of c (pade_robust.f90:347-352)
-__device__ void pr_build(double2 *A, const double2 *cc, int m, int n, int l, double d) {
+template <int G> __device__ void pr_build(double2 *A, const double2 *cc, int m, int n, int l, double d) {
   __syncwarp();
   for (int i = 0; i < n; ++i) {
     const int k = m + 1 + i - l;
     const double2 v = (l <= n && k >= 0) ? cc[k] : mk(0.0, 0.0);
-    A[i * kPrLanes + l] = mk(v.x * d, v.y * d);
+    A[i * G + l] = mk(v.x * d, v.y * d);
   }
   __syncwarp();
 }
 
-// number of singular values of A (rows x cols, rows <= 32) above tol:
+// Whether the columns of A, part way through Jacobi, already fix the number of
+// singular values above tol, and that number.  Columns of norm above 3 tol
+// with all cosines below 1/(2 k) (k of them) have a smallest singular value
+// of at least their smallest norm times sqrt(1/2), which is above 2 tol; the
+// others together, below tol/2 in Frobenius norm, move no singular value by
+// more than that.  The rotations still to come keep the singular values up to
+// their rounding, a few 1e-16 of the matrix, against tol = 1e-14 ||c||, so
+// they cannot carry one across tol.
+template <int G> __device__ bool pr_decided(const double2 *A, int rows, int cols, int l,
+                                            double tol, int &rho) {
+  double rest = 0.0;
+  uint32_t big = 0;
+  for (int i = 0; i < cols; ++i) {
+    const double2 a = l < rows ? A[i * G + l] : mk(0.0, 0.0);
+    const double s = lanes::sum<G>(cabs2(a));
+    if (s > 9.0 * tol * tol) big |= 1u << i;
+    else rest += s;
+  }
+  if (!(rest < 0.25 * tol * tol)) return false;
+  const int k = __popc(big);
+  const double lim = 0.25 / ((double)k * k);
+  for (uint32_t m = big; m; m &= m - 1) {
+    const int p = __ffs(m) - 1;
+    const double2 ap = l < rows ? A[p * G + l] : mk(0.0, 0.0);
+    const double al = lanes::sum<G>(cabs2(ap));
+    for (uint32_t m2 = m & (m - 1); m2; m2 &= m2 - 1) {
+      const int q = __ffs(m2) - 1;
+      const double2 aq = l < rows ? A[q * G + l] : mk(0.0, 0.0);
+      double2 g = mk(0.0, 0.0);
+      cmacc(g, ap, aq);
+      g = mk(lanes::sum<G>(g.x), lanes::sum<G>(g.y));
+      if (!(cabs2(g) < lim * al * lanes::sum<G>(cabs2(aq)))) return false;
+    }
+  }
+  rho = k;
+  return true;
+}
+
+// number of singular values of A (rows x cols, rows <= G) above tol:
 // one-sided (Hestenes) Jacobi orthogonalises the columns, whose norms are
-// then the singular values.  Each lane touches only its own row of A.
-__device__ int pr_rank(double2 *A, int rows, int cols, int l, double tol) {
+// then the singular values.  Each lane touches only its own row of A.  It
+// stops once the number is certain; where a singular value comes near tol it
+// runs to convergence.
+template <int G> __device__ int pr_rank(double2 *A, int rows, int cols, int l, double tol) {
   const double ctol = sqrt((double)rows) * kDblEps;
   for (int sweep = 0; sweep < kPrSweeps; ++sweep) {
     int rot = 0;
-    for (int p = 0; p + 1 < cols; ++p)
+    for (int p = 0; p + 1 < cols; ++p) {
+      // column p stays in registers over its pairs; the next column is read,
+      // and its norm summed, ahead of the pair that needs them
+      double2 ap = l < rows ? A[p * G + l] : mk(0.0, 0.0);
+      double2 aq = l < rows ? A[(p + 1) * G + l] : mk(0.0, 0.0);
+      double al = lanes::sum<G>(cabs2(ap)), be = lanes::sum<G>(cabs2(aq));
+      bool turned = false;
       for (int q = p + 1; q < cols; ++q) {
-        const double2 ap = l < rows ? A[p * kPrLanes + l] : mk(0.0, 0.0);
-        const double2 aq = l < rows ? A[q * kPrLanes + l] : mk(0.0, 0.0);
-        const double al = gsum(cabs2(ap)), be = gsum(cabs2(aq));
         double2 gm = mk(0.0, 0.0);
         cmacc(gm, ap, aq);                                   // conj(a_p) a_q
-        gm = mk(gsum(gm.x), gsum(gm.y));
-        const double g = hypot(gm.x, gm.y);
-        if (!(g > ctol * sqrt(al) * sqrt(be))) continue;    // uniform over the group
-        ++rot;
-        // a_q~ = a_q conj(g)/|g| makes a_p^H a_q~ = |g| real; then the real
-        // rotation with t^2 + 2 zeta t - 1 = 0, |t| <= 1
-        const double zeta = (be - al) / (2.0 * g);
-        const double az = fabs(zeta);
-        const double t = az > 1e150 ? 0.5 / zeta : copysign(1.0, zeta) / (az + sqrt(1.0 + zeta * zeta));
-        const double cs = 1.0 / sqrt(1.0 + t * t), sn = cs * t;
-        const double2 ph = mk(gm.x / g, -gm.y / g);
-        const double2 aqt = cmul(aq, ph);
-        if (l < rows) {
-          A[p * kPrLanes + l] = mk(cs * ap.x - sn * aqt.x, cs * ap.y - sn * aqt.y);
-          A[q * kPrLanes + l] = mk(sn * ap.x + cs * aqt.x, sn * ap.y + cs * aqt.y);
+        gm = mk(lanes::sum<G>(gm.x), lanes::sum<G>(gm.y));
+        const double g2 = cabs2(gm);
+        const double2 an = q + 1 < cols && l < rows ? A[(q + 1) * G + l] : mk(0.0, 0.0);
+        const double bn = lanes::sum<G>(cabs2(an));
+        // far from the threshold its roots are not needed
+        const double c2 = ctol * ctol * al * be;
+        const double g = g2 < 0.5 * c2 ? 0.0 : hypot(gm.x, gm.y);
+        if (g2 > 2.0 * c2 || g > ctol * sqrt(al) * sqrt(be)) {  // uniform over the group
+          ++rot;
+          turned = true;
+          // a_q~ = a_q conj(g)/|g| makes a_p^H a_q~ = |g| real; then the real
+          // rotation with t^2 + 2 zeta t - 1 = 0, |t| <= 1
+          const double zeta = (be - al) / (2.0 * g);
+          const double az = fabs(zeta);
+          const double t =
+              az > 1e150 ? 0.5 / zeta : copysign(1.0, zeta) / (az + sqrt(1.0 + zeta * zeta));
+          const double cs = 1.0 / sqrt(1.0 + t * t), sn = cs * t;
+          const double2 ph = mk(gm.x / g, -gm.y / g);
+          const double2 aqt = cmul(aq, ph);
+          if (l < rows) A[q * G + l] = mk(sn * ap.x + cs * aqt.x, sn * ap.y + cs * aqt.y);
+          ap = mk(cs * ap.x - sn * aqt.x, cs * ap.y - sn * aqt.y);
+          al = lanes::sum<G>(cabs2(ap));
         }
+        aq = an;
+        be = bn;
       }
+      if (turned && l < rows) A[p * G + l] = ap;
+    }
     if (rot == 0) break;
+    int sure;
+    if (pr_decided<G>(A, rows, cols, l, tol, sure)) return sure;
   }
   int rho = 0;
   for (int i = 0; i < cols; ++i) {
-    const double2 a = l < rows ? A[i * kPrLanes + l] : mk(0.0, 0.0);
-    if (sqrt(gsum(cabs2(a))) > tol) ++rho;
+    const double2 a = l < rows ? A[i * G + l] : mk(0.0, 0.0);
+    if (sqrt(lanes::sum<G>(cabs2(a))) > tol) ++rho;
   }
   return rho;
+}
+
+// The number of singular values of A above tol where a column-pivoted QR
+// settles it, else -1 (Jacobi decides then; A is overwritten).  After k steps
+// sigma_{k+1} is at most the Frobenius norm of what is left, required below
+// tol / 2, and sigma_k at least 3 r_kk / sqrt(4^k + 6 k - 1) (Faddeev,
+// Kublanovskaya and Faddeeva; the columns are pivoted), required above 2 tol.
+// The margins cover the rounding of either algorithm, a few 1e-16 ||A||
+// against tol = 1e-14 ||c||.
+template <int G> __device__ int pr_rank_qr(double2 *A, int rows, int cols, int l, double tol) {
+  // lane j keeps the squared norm of column j (-1: taken)
+  double nj = -1.0, rest = 0.0;
+  for (int j = 0; j < cols; ++j) {
+    const double s = lanes::sum<G>(l < rows ? cabs2(A[j * G + l]) : 0.0);
+    if (l == j) nj = s;
+    rest += s;
+  }
+  double rkk = 0.0;
+  int k = 0;
+  while (k < cols && !(rest < 0.25 * tol * tol)) {
+    const double big = lanes::max<G>(nj);
+    const int p = lanes::min<G>(nj == big ? l : G - 1);
+    if (!(big > 0.0) || k >= 26) return -1;  // nothing left, NaN, or no use for the bound
+    if (l == p) nj = -1.0;
+    rkk = sqrt(big);
+    const double inv = 1.0 / rkk;
+    double2 qv = l < rows ? A[p * G + l] : mk(0.0, 0.0);
+    qv = mk(qv.x * inv, qv.y * inv);
+    ++k;
+    rest = 0.0;
+    const uint64_t left = __ballot(nj >= 0.0) >> ((threadIdx.x & 63) / G * G);
+    for (uint32_t m = (uint32_t)left & (uint32_t)((1ull << G) - 1); m; m &= m - 1) {
+      const int j = __ffs(m) - 1;
+      double2 a = l < rows ? A[j * G + l] : mk(0.0, 0.0), g = mk(0.0, 0.0);
+      cmacc(g, qv, a);
+      g = mk(lanes::sum<G>(g.x), lanes::sum<G>(g.y));
+      a = csub(a, cmul(qv, g));
+      if (l < rows) A[j * G + l] = a;
+      const double s = lanes::sum<G>(cabs2(a));
+      if (l == j) nj = s;
+      rest += s;
+    }
+  }
+  if (k == 0) return 0;
+  // sqrt(4^k + 6 k - 1) < 2^k (1 + 6 k / 4^k)
+  const double f = (double)(1u << k);
+  return 3.0 * rkk > 2.0 * tol * f * (1.0 + 6.0 * k / (f * f)) ? k : -1;
 }
 
 // Householder QR of A (rows x cols, rows = cols + 1 <= 31) in place, in the
 // conventions of ZGEQR2/ZLARFG: H_k = I - tau_k v_k v_k^H with v_k(k) = 1,
 // beta = -sign(Re alpha) ||(alpha, x)||; R on and above the diagonal, v_k
 // below it, tau_k in tau[k]
-__device__ void pr_qr(double2 *A, double2 *tau, int rows, int cols, int l) {
+template <int G> __device__ void pr_qr(double2 *A, double2 *tau, int rows, int cols, int l) {
   for (int k = 0; k < cols; ++k) {
     __syncwarp();
-    const double2 alpha = A[k * kPrLanes + k];
+    const double2 alpha = A[k * G + k];
     const bool below = l > k && l < rows;
-    const double2 x = below ? A[k * kPrLanes + l] : mk(0.0, 0.0);
-    const double xn2 = gsum(cabs2(x));
+    const double2 x = below ? A[k * G + l] : mk(0.0, 0.0);
+    const double xn2 = lanes::sum<G>(cabs2(x));
     double2 tk = mk(0.0, 0.0);
     if (!(xn2 == 0.0 && alpha.y == 0.0)) {
       const double beta = -copysign(sqrt(alpha.x * alpha.x + alpha.y * alpha.y + xn2), alpha.x);
       tk = mk((beta - alpha.x) / beta, -alpha.y / beta);
       const double2 sc = cdiv(mk(1.0, 0.0), mk(alpha.x - beta, alpha.y));
       const double2 v = l == k ? mk(1.0, 0.0) : (below ? cmul(x, sc) : mk(0.0, 0.0));
-      if (below) A[k * kPrLanes + l] = v;
-      if (l == k) A[k * kPrLanes + k] = mk(beta, 0.0);
+      if (below) A[k * G + l] = v;
+      if (l == k) A[k * G + k] = mk(beta, 0.0);
       // H_k^H = I - conj(tau_k) v v^H on the columns right of k
       const double2 ct = cconj(tk);
       for (int j = k + 1; j < cols; ++j) {
         const bool act = l >= k && l < rows;
-        const double2 a = act ? A[j * kPrLanes + l] : mk(0.0, 0.0);
+        const double2 a = act ? A[j * G + l] : mk(0.0, 0.0);
         double2 s = mk(0.0, 0.0);
         cmacc(s, v, a);
-        s = mk(gsum(s.x), gsum(s.y));
-        if (act) A[j * kPrLanes + l] = csub(a, cmul(ct, cmul(v, s)));
+        s = mk(lanes::sum<G>(s.x), lanes::sum<G>(s.y));
+        if (act) A[j * G + l] = csub(a, cmul(ct, cmul(v, s)));
       }
     }
     if (l == 0) tau[k] = tk;
@@ -226,14 +321,14 @@ __device__ void pr_qr(double2 *A, double2 *tau, int rows, int cols, int l) {
 
 // row l of Q e_{rows-1}, Q = H_0 H_1 ... H_{cols-1} (the last column of the
 // full Q of ZUNGQR)
-__device__ double2 pr_qlast(const double2 *A, const double2 *tau, int rows, int cols, int l) {
+template <int G> __device__ double2 pr_qlast(const double2 *A, const double2 *tau, int rows, int cols, int l) {
   double2 y = l == rows - 1 ? mk(1.0, 0.0) : mk(0.0, 0.0);
   for (int k = cols - 1; k >= 0; --k) {
     const double2 v = l == k ? mk(1.0, 0.0)
-                             : ((l > k && l < rows) ? A[k * kPrLanes + l] : mk(0.0, 0.0));
+                             : ((l > k && l < rows) ? A[k * G + l] : mk(0.0, 0.0));
     double2 s = mk(0.0, 0.0);
     cmacc(s, v, y);
-    s = mk(gsum(s.x), gsum(s.y));
+    s = mk(lanes::sum<G>(s.x), lanes::sum<G>(s.y));
     y = csub(y, cmul(tau[k], cmul(v, s)));
   }
   return y;
@@ -243,8 +338,15 @@ __device__ double2 pr_qlast(const double2 *A, const double2 *tau, int rows, int 
 // the values on the circle z_f = R e^{2 pi i f / N} and receives
 // [m, n, a_0..a_m, b_0..b_n, 0, ...] (the reference leaves whatever was there
 // beyond the coefficients; pade_eval_robust never reads it)
-__global__ __launch_bounds__(kPrLanes *kPrGroups) void k_pade_robust_coeffs(
-    int64_t ne, int N, double radius, int nmax, double2 *__restrict__ w) {
+//
+// EXACT: ranks by Jacobi.  Otherwise ranks by pr_rank_qr, and an element
+// where that leaves one open goes, untouched, to the list `open` (open[0]
+// their number), which a second launch with EXACT works off; with `open` null
+// an EXACT launch takes every element.
+template <int G, bool EXACT>
+__global__ __launch_bounds__(kPrBlock) void k_pade_robust_coeffs(
+    int64_t ne, int N, double radius, int nmax, double2 *__restrict__ w,
+    int32_t *__restrict__ open) {
   extern __shared__ double2 pr_lds[];
   __shared__ double2 tw[kMaxPade];
   for (int t = threadIdx.x; t < N; t += blockDim.x) {
@@ -253,15 +355,16 @@ __global__ __launch_bounds__(kPrLanes *kPrGroups) void k_pade_robust_coeffs(
     tw[t] = mk(c, s);
   }
   __syncthreads();
-  const int grp = threadIdx.x / kPrLanes, l = threadIdx.x % kPrLanes;
-  const int64_t e = (int64_t)blockIdx.x * (blockDim.x / kPrLanes) + grp;
-  if (e >= ne) return;
-  double2 *fa = pr_lds + (size_t)grp * pr_group_lds(nmax);   // f, later a
-  double2 *cc = fa + kMaxPade;
-  double2 *bv = cc + kMaxPade;
-  double2 *tau = bv + kPrLanes;
-  double2 *A = tau + kPrLanes;
-  for (int j = l; j < N; j += kPrLanes) fa[j] = w[(int64_t)j * ne + e];
+  const int grp = threadIdx.x / G, l = threadIdx.x % G;
+  const int64_t at = (int64_t)blockIdx.x * (blockDim.x / G) + grp;
+  if (at >= (EXACT && open ? open[0] : ne)) return;
+  const int64_t e = EXACT && open ? open[1 + at] : at;
+  double2 *cc = pr_lds + (size_t)grp * pr_group_lds<G>(nmax);
+  double2 *bv = cc + 2 * G;
+  double2 *tau = bv + G;
+  double2 *A = tau + G;
+  double2 *fa = A;  // f before the matrix, a after it
+  for (int j = l; j < N; j += G) fa[j] = w[(int64_t)j * ne + e];
   __syncwarp();
 
   int m = N / 2 - 2, n = m;            // the (n, n) start, pade_coeff_robust :146-147
@@ -271,10 +374,14 @@ __global__ __launch_bounds__(kPrLanes *kPrGroups) void k_pade_robust_coeffs(
   double nrm = 0.0;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int k = l + h * kPrLanes;
+    const int k = l + h * G;
     double2 acc = mk(0.0, 0.0);
     if (k < nd) {
-      for (int j = 0; j < N; ++j) cmac(acc, fa[j], tw[(j * k) % N]);
+      for (int j = 0, t = 0; j < N; ++j) {  // t = j k mod N
+        cmac(acc, fa[j], tw[t]);
+        t += k;
+        t -= t >= N ? N : 0;
+      }
       acc = mk(acc.x * (1.0 / N), acc.y * (1.0 / N));
       if (fabs(radius - 1.0) > kPrTol) {
         double r = 1.0;
@@ -286,30 +393,30 @@ __global__ __launch_bounds__(kPrLanes *kPrGroups) void k_pade_robust_coeffs(
     nrm += cabs2(acc);
   }
   {
-    const double tol = kPrTol * sqrt(gsum(nrm));   // near-zero coefficients dropped
+    const double tol = kPrTol * sqrt(lanes::sum<G>(nrm));   // near-zero coefficients dropped
     double im = 0.0;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       if (cabsd(ck[h]) < tol) ck[h] = mk(0.0, 0.0);
       im = fmax(im, fabs(ck[h].y));
     }
-    if (gmax(im) < tol) {                           // real functions made real
+    if (lanes::max<G>(im) < tol) {                           // real functions made real
       ck[0].y = 0.0;
       ck[1].y = 0.0;
     }
   }
   cc[l] = ck[0];
-  cc[l + kPrLanes] = ck[1];
-  const double abs_tol = kPrTol * sqrt(gsum(cabs2(ck[0]) + cabs2(ck[1])));   // :276
+  cc[l + G] = ck[1];
+  const double abs_tol = kPrTol * sqrt(lanes::sum<G>(cabs2(ck[0]) + cabs2(ck[1])));   // :276
   double cmax = 0.0, cmax_m = 0.0;
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
-    const int k = l + h * kPrLanes;
+    const int k = l + h * G;
     cmax = fmax(cmax, cabsd(ck[h]));
     if (k <= m) cmax_m = fmax(cmax_m, cabsd(ck[h]));
   }
-  cmax = gmax(cmax);
-  cmax_m = gmax(cmax_m);
+  cmax = lanes::max<G>(cmax);
+  cmax_m = lanes::max<G>(cmax_m);
   __syncwarp();
 
   double2 a = mk(0.0, 0.0), b = mk(0.0, 0.0);      // row l of a and of b
@@ -321,8 +428,13 @@ __global__ __launch_bounds__(kPrLanes *kPrGroups) void k_pade_robust_coeffs(
   } else {
     // diagonal hopping (:318-363): while rank(C) < n, shrink m and n
     while (n > 0) {
-      pr_build(A, cc, m, n, l, 1.0);
-      const int rho = pr_rank(A, n + 1, n, l, abs_tol);
+      pr_build<G>(A, cc, m, n, l, 1.0);
+      const int rho = EXACT ? pr_rank<G>(A, n + 1, n, l, abs_tol)
+                            : pr_rank_qr<G>(A, n + 1, n, l, abs_tol);
+      if (!EXACT && rho < 0) {
+        if (l == 0) open[1 + atomicAdd(open, 1)] = (int32_t)e;
+        return;
+      }
       if (rho == n) break;
       m -= n - rho;
       n = rho;
@@ -334,15 +446,15 @@ __global__ __launch_bounds__(kPrLanes *kPrGroups) void k_pade_robust_coeffs(
       // null vector of C (a unit vector, up to phase the one of ZGESDD) gives
       // the weights D = |v| + sqrt(eps); then b = D q_{n+1} of the QR of
       // (C D)^T, normalised (:366-386)
-      pr_build(A, cc, m, n, l, 1.0);
-      pr_qr(A, tau, n + 1, n, l);
-      double2 y = pr_qlast(A, tau, n + 1, n, l);
+      pr_build<G>(A, cc, m, n, l, 1.0);
+      pr_qr<G>(A, tau, n + 1, n, l);
+      double2 y = pr_qlast<G>(A, tau, n + 1, n, l);
       const double d = l <= n ? cabsd(y) + kSqrtEps : 0.0;
-      pr_build(A, cc, m, n, l, d);
-      pr_qr(A, tau, n + 1, n, l);
-      y = pr_qlast(A, tau, n + 1, n, l);
+      pr_build<G>(A, cc, m, n, l, d);
+      pr_qr<G>(A, tau, n + 1, n, l);
+      y = pr_qlast<G>(A, tau, n + 1, n, l);
       b = mk(d * y.x, d * y.y);
-      const double bn = sqrt(gsum(cabs2(b)));
+      const double bn = sqrt(lanes::sum<G>(cabs2(b)));
       b = mk(b.x / bn, b.y / bn);
       bv[l] = b;
       __syncwarp();
@@ -350,8 +462,8 @@ __global__ __launch_bounds__(kPrLanes *kPrGroups) void k_pade_robust_coeffs(
       if (l <= m)
         for (int j = 0; j <= min(l, n); ++j) cmac(a, cc[l - j], bv[j]);
       // leading zeros of b (and a) dropped (:392-408)
-      int lam = gmini((l <= n && cabsd(b) > kPrTol) ? l : kPrLanes);
-      if (lam == kPrLanes) lam = 0;
+      int lam = lanes::min<G>((l <= n && cabsd(b) > kPrTol) ? l : G);
+      if (lam == G) lam = 0;
       if (lam > 0) {
         fa[l] = a;
         __syncwarp();
@@ -362,7 +474,7 @@ __global__ __launch_bounds__(kPrLanes *kPrGroups) void k_pade_robust_coeffs(
         __syncwarp();
       }
       // trailing zeros of b dropped (:411-420)
-      const int last = gmaxi((l <= n && cabsd(b) > kPrTol) ? l : -1);
+      const int last = lanes::max<G>((l <= n && cabsd(b) > kPrTol) ? l : -1);
       if (last != n) {
         n = last;
         if (l > n) b = mk(0.0, 0.0);
@@ -370,7 +482,7 @@ __global__ __launch_bounds__(kPrLanes *kPrGroups) void k_pade_robust_coeffs(
     }
   }
   // trailing zeros of a dropped (:425-434), then a and b over b_0 (:437-438)
-  const int last_a = zero ? m : gmaxi((l <= m && cabsd(a) > abs_tol) ? l : -1);
+  const int last_a = zero ? m : lanes::max<G>((l <= m && cabsd(a) > abs_tol) ? l : -1);
   if (last_a != m) {
     m = last_a;
     if (l > m) a = mk(0.0, 0.0);
@@ -385,7 +497,7 @@ __global__ __launch_bounds__(kPrLanes *kPrGroups) void k_pade_robust_coeffs(
   bv[l] = b;
   __syncwarp();
   // slices: 0 -> m, 1 -> n, 2..2+m -> a, 3+m..3+m+n -> b, the rest 0
-  for (int s = l; s < N; s += kPrLanes) {
+  for (int s = l; s < N; s += G) {
     double2 v = mk(0.0, 0.0);
     if (s == 0) v = mk((double)m, 0.0);
     else if (s == 1) v = mk((double)n, 0.0);
@@ -607,10 +719,40 @@ extern "C" int sgw_analytic_coeff(int32_t model, double thres, int32_t num_g, in
                     "pade_coeff_robust: frequencies must span circle in the complex plane");
       SGW_REQUIRE(radius > 0.0, SGW_E_ARG, "pade_robust: radius in the complex plane must be > 0");
       const int nmax = nfreq / 2 - 2;
-      const int per = (int)sizeof(double2) * pr_group_lds(nmax);   // <= 18432 bytes
-      const int gpb = std::min(kPrGroups, kPrLdsMax / per);
-      k_pade_robust_coeffs<<<(unsigned)((ne + gpb - 1) / gpb), kPrLanes * gpb, (size_t)gpb * per,
-                             st>>>(ne, nfreq, radius, nmax, w);
+      DevBuf<int32_t> open;
+      auto go = [&](auto group) {
+        constexpr int G = decltype(group)::value;
+        const int bytes = (int)sizeof(double2) * pr_group_lds<G>(nmax);   // <= 18432
+        const int per = std::min(kPrBlock / G, kPrLdsMax / bytes);
+        const unsigned grid = (unsigned)((ne + per - 1) / per);
+        if (!open.p) {
+          k_pade_robust_coeffs<G, true><<<grid, G * per, (size_t)per * bytes, st>>>(
+              ne, nfreq, radius, nmax, w, nullptr);
+          return;
+        }
+        k_pade_robust_coeffs<G, false><<<grid, G * per, (size_t)per * bytes, st>>>(
+            ne, nfreq, radius, nmax, w, open.p);
+        // as many groups as elements might be open: those past the list's end leave at once
+        k_pade_robust_coeffs<G, true><<<grid, G * per, (size_t)per * bytes, st>>>(
+            ne, nfreq, radius, nmax, w, open.p);
+      };
+      // the list of open elements; a stream under capture takes every element
+      // through Jacobi instead (no allocation there)
+      hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+      if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
+        (void)hipGetLastError();
+        cap = hipStreamCaptureStatusActive;
+      }
+      if (cap == hipStreamCaptureStatusNone && ne < (1ll << 31) - 1) {
+        open.alloc((size_t)ne + 1);
+        SGW_HIP(hipMemsetAsync(open.p, 0, sizeof(int32_t), st));
+      }
+      if (nfreq <= kPrSmallMax) go(std::integral_constant<int, 16>{});
+      else go(std::integral_constant<int, 32>{});
+      if (open.p) {
+        SGW_HIP(hipGetLastError());
+        SGW_HIP(hipStreamSynchronize(st));  // the list is freed here
+      }
     } else if (model == SGW_AAA_APPROX || model == SGW_AAA_POLE) {
       // aaa_generate per element on the symmetrised mesh (analytic.f90:162-199)
       const Mesh m = make_mesh(nfreq, h_z, h_src);
