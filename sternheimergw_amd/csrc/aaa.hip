@@ -3,8 +3,8 @@
 // Trefethen, SIAM J. Sci. Comput. 40 (2018) A1494) for every (G, G')
 // element, and the pole-residue form of analytic.f90:389-427.
 //
-// One wavefront per element, lane i on mesh point i (at most 64 points).
-// Per greedy step the Loewner submatrix (rows: the points that are not
+// Half a wavefront per element, lane l on mesh points l and l + 32 (at most 64
+// points).  Per greedy step the Loewner submatrix (rows: the points that are not
 // support points, columns: the support points in mesh order) sits in LDS
 // column by column; its last right singular vector comes from one-sided
 // (Hestenes) Jacobi with the rotations accumulated in V (the reference calls
@@ -14,48 +14,46 @@
 // finite eigenvalues of the reference's arrowhead pencil (ZGGEV there),
 // found together by Aberth-Ehrlich iteration, one lane per zero.
 #include <algorithm>
+#include <climits>
 #include <cmath>
 
 #include "aaa.h"
+#include "lanes.h"
 #include "sgw_internal.h"
 
 namespace sgw {
 namespace {
 
 constexpr int kAaaMax = 64;                             // mesh points
-constexpr int kVs = 32;                                 // column stride of V
 constexpr double kEps6 = 1e-6, kEps14 = 1e-14;
 constexpr double kDblEpsA = 2.220446049250313e-16;
 constexpr int kSweeps = 40, kAberthIters = 500;
 
-__device__ inline double wsum(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-  return v;
+constexpr int kGrp = 32;                                // lanes per element
+
+// sums and extrema over the mesh points or matrix rows of an element, H to a
+// lane; the order is that of a 64-lane butterfly (lane l and l + 32 first)
+template <int H> __device__ inline double wsum(const double (&v)[H]) {
+  return lanes::sum<kGrp>(H == 2 ? v[0] + v[H - 1] : v[0]);
 }
-__device__ inline double wmax(double v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
-  return v;
+template <int H> __device__ inline double wmax(const double (&v)[H]) {
+  return lanes::max<kGrp>(H == 2 ? fmax(v[0], v[H - 1]) : v[0]);
 }
-__device__ inline double2 wsum2(double2 v) { return mk(wsum(v.x), wsum(v.y)); }
+template <int H> __device__ inline double2 wsum2(const double2 (&v)[H]) {
+  double re[H], im[H];
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    re[h] = v[h].x;
+    im[h] = v[h].y;
+  }
+  return mk(wsum<H>(re), wsum<H>(im));
+}
+// this group's half of a wavefront ballot
+__device__ inline uint32_t gballot(bool c) {
+  return (uint32_t)(__ballot(c) >> (threadIdx.x & 32));
+}
 __device__ inline double cabs2a(double2 a) { return a.x * a.x + a.y * a.y; }
 __device__ inline double cabsa(double2 a) { return hypot(a.x, a.y); }
-
-// (value, index) of the largest value over the wavefront, the lowest index
-// among equal ones (MAXLOC); every lane gets the same pair
-__device__ inline int wargmax(double v, int i) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) {
-    const double v2 = __shfl_xor(v, o, 64);
-    const int i2 = __shfl_xor(i, o, 64);
-    if (v2 > v || (v2 == v && i2 < i)) {
-      v = v2;
-      i = i2;
-    }
-  }
-  return i;
-}
 
 __device__ inline uint64_t below(int l) { return l == 0 ? 0ull : (~0ull >> (64 - l)); }
 
@@ -90,107 +88,179 @@ struct AaaMesh {
   int src[kAaaMax];
 };
 
-// LDS per wavefront (double2 units): A (64 x mcap), V (32 x mcap), pos, val,
-// wgt, lam (64 each)
-__host__ __device__ inline int aaa_lds(int mcap) { return (kAaaMax + kVs) * mcap + 4 * kAaaMax; }
+// LDS per element (double2 units): A (M x mcap), V (mcap x mcap), pos, val,
+// wgt, lam (mcap each)
+__host__ __device__ inline int aaa_lds(int M, int mcap) { return (M + mcap + 4) * mcap; }
 
 // model 4: slices [pos (mmax), val (mmax), wgt (mmax), 0...], mmax = max_point;
 // model 5: [poles, 0..., residues, 0...] in halves of N / 2.
 // status[0] = 1: a model-5 element needed more than mcap support points;
 // status[1] = 1: more relevant poles than N / 2 (pole_correction's error)
+//
+// Bound: the dependent FP64 chains of the Jacobi pairs.  H mesh points and
+// matrix rows to a lane; two elements share a wavefront, and the group sums
+// are vector instructions (lanes.h), so the rows of a pair wait for no LDS
+// permute.  400 x 400 elements, 35 points, at most 11 support points: 18.2 ms,
+// against 42.4 with one wavefront per element and LDS-permute sums.
+template <int H>
 __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh mesh, double thres,
                                                   int model, int max_point, int mcap,
                                                   double2 *__restrict__ w,
                                                   int32_t *__restrict__ status) {
   extern __shared__ double2 aaa_smem[];
-  const int64_t e = blockIdx.x;
-  const int l = threadIdx.x;
-  double2 *A = aaa_smem;
-  double2 *V = A + kAaaMax * mcap;
-  double2 *pos = V + kVs * mcap;
-  double2 *val = pos + kAaaMax;
-  double2 *wgt = val + kAaaMax;
-  double2 *lam = wgt + kAaaMax;
-  const bool pt = l < M;
-  const double2 zl = pt ? mesh.z[l] : mk(0.0, 0.0);
-  const double2 fl = pt ? w[(int64_t)mesh.src[l] * ne + e] : mk(0.0, 0.0);
+  const int64_t e = (int64_t)blockIdx.x * 2 + threadIdx.x / kGrp;
+  const int l = threadIdx.x % kGrp;
+  if (e >= ne) return;
+  double2 *A = aaa_smem + (size_t)(threadIdx.x / kGrp) * aaa_lds(M, mcap);
+  double2 *V = A + M * mcap;
+  double2 *pos = V + mcap * mcap;
+  double2 *val = pos + mcap;
+  double2 *wgt = val + mcap;
+  double2 *lam = wgt + mcap;
+  const double2 zero = mk(0.0, 0.0);
+  const uint64_t all = M == 64 ? ~0ull : (1ull << M) - 1;
+  double2 zl[H], fl[H], fit[H];
+  bool pt[H], sup[H];
+  double d[H];
+#pragma unroll
+  for (int h = 0; h < H; ++h) {
+    const int i = l + kGrp * h;
+    pt[h] = i < M;
+    sup[h] = false;
+    zl[h] = pt[h] ? mesh.z[i] : zero;
+    fl[h] = pt[h] ? w[(int64_t)mesh.src[i] * ne + e] : zero;
+    d[h] = pt[h] ? cabsa(fl[h]) : 0.0;
+  }
   // setup_work_type (:119-148)
-  const double thres_abs = thres * wmax(pt ? cabsa(fl) : 0.0);
-  const double2 sumf = wsum2(fl);
-  double2 fit = mk(sumf.x / M, sumf.y / M);
-  bool sup = false;
+  const double thres_abs = thres * wmax<H>(d);
+  const double2 sumf = wsum2<H>(fl);
+#pragma unroll
+  for (int h = 0; h < H; ++h) fit[h] = mk(sumf.x / M, sumf.y / M);
   int m = 0;
   const int mp = max_point;
   for (;;) {
-    // update_support_point (:178-187)
-    const int j = wargmax(pt ? cabsa(csub(fl, fit)) : -1.0, l);
-    if (l == j) {
-      fit = fl;
-      sup = true;
+    // update_support_point (:178-187): the first point of largest |f - fit|
+#pragma unroll
+    for (int h = 0; h < H; ++h) d[h] = pt[h] ? cabsa(csub(fl[h], fit[h])) : -1.0;
+    const double dmax = wmax<H>(d);
+    int first = INT_MAX;
+#pragma unroll
+    for (int h = H - 1; h >= 0; --h)
+      if (d[h] == dmax) first = l + kGrp * h;
+    const int j = lanes::min<kGrp>(first);
+    uint64_t smask = 0;
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      if (l + kGrp * h == j) {
+        fit[h] = fl[h];
+        sup[h] = true;
+      }
+      smask |= (uint64_t)gballot(sup[h]) << (kGrp * h);
     }
     ++m;
-    const uint64_t smask = __ballot(sup) & (M == 64 ? ~0ull : (1ull << M) - 1);
-    const uint64_t rmask = ~smask & (M == 64 ? ~0ull : (1ull << M) - 1);
+    smask &= all;
+    const uint64_t rmask = ~smask & all;
     const int nrows = M - m;
     if (m > mcap) {  // the device keeps at most mcap support points
       if (l == 0) status[0] = 1;
       break;
     }
     __syncwarp();
-    if (sup) {
-      const int c = __popcll(smask & below(l));
-      pos[c] = zl;
-      val[c] = fl;
-    }
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+      if (sup[h]) {
+        const int c = __popcll(smask & below(l + kGrp * h));
+        pos[c] = zl[h];
+        val[c] = fl[h];
+      }
     __syncwarp();
     // determine_weight (:205-225): the Loewner submatrix, rows = the other
     // points in mesh order, columns = the support points in mesh order
-    const int r = __popcll(rmask & below(l));
-    if (pt && !sup)
-      for (int c = 0; c < m; ++c) A[c * kAaaMax + r] = cdiv(csub(fl, val[c]), csub(zl, pos[c]));
+#pragma unroll
+    for (int h = 0; h < H; ++h) {
+      const int r = __popcll(rmask & below(l + kGrp * h));
+      if (pt[h] && !sup[h])
+        for (int c = 0; c < m; ++c)
+          A[c * M + r] = cdiv(csub(fl[h], val[c]), csub(zl[h], pos[c]));
+    }
     if (l < m)
-      for (int c = 0; c < m; ++c) V[c * kVs + l] = mk(l == c ? 1.0 : 0.0, 0.0);
+      for (int c = 0; c < m; ++c) V[c * mcap + l] = mk(l == c ? 1.0 : 0.0, 0.0);
     __syncwarp();
+    auto column = [&](int c, double2 (&a)[H]) {
+#pragma unroll
+      for (int h = 0; h < H; ++h) a[h] = l + kGrp * h < nrows ? A[c * M + l + kGrp * h] : zero;
+    };
+    auto norm2 = [&](const double2 (&a)[H]) {
+      double s[H];
+#pragma unroll
+      for (int h = 0; h < H; ++h) s[h] = cabs2a(a[h]);
+      return wsum<H>(s);
+    };
     int cmin = m - 1;  // an empty submatrix: V = I, the weight is e_m
     if (nrows > 0) {
       const double ctol = sqrt((double)nrows) * kDblEpsA;
       for (int sweep = 0; sweep < kSweeps; ++sweep) {
         int rot = 0;
-        for (int p = 0; p + 1 < m; ++p)
+        for (int p = 0; p + 1 < m; ++p) {
+          // column p stays in registers over its pairs
+          double2 ap[H], aq[H];
+          column(p, ap);
+          double2 vp = l < m ? V[p * mcap + l] : zero;
+          double al = norm2(ap);
+          bool turned = false;
           for (int q = p + 1; q < m; ++q) {
-            const double2 ap = l < nrows ? A[p * kAaaMax + l] : mk(0.0, 0.0);
-            const double2 aq = l < nrows ? A[q * kAaaMax + l] : mk(0.0, 0.0);
-            const double al = wsum(cabs2a(ap)), be = wsum(cabs2a(aq));
-            double2 gm = mk(0.0, 0.0);
-            cmacc(gm, ap, aq);
-            gm = wsum2(gm);
+            column(q, aq);
+            const double be = norm2(aq);
+            double2 gh[H];
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+              gh[h] = zero;
+              cmacc(gh[h], ap[h], aq[h]);
+            }
+            const double2 gm = wsum2<H>(gh);
+            // far from the threshold its roots are not needed
+            const double g2 = cabs2a(gm), c2 = ctol * ctol * al * be;
+            if (g2 < 0.5 * c2) continue;
             const double g = hypot(gm.x, gm.y);
-            if (!(g > ctol * sqrt(al) * sqrt(be))) continue;
+            if (!(g2 > 2.0 * c2) && !(g > ctol * sqrt(al) * sqrt(be))) continue;
             ++rot;
+            turned = true;
             const double zeta = (be - al) / (2.0 * g);
             const double az = fabs(zeta);
             const double t =
                 az > 1e150 ? 0.5 / zeta : copysign(1.0, zeta) / (az + sqrt(1.0 + zeta * zeta));
             const double cs = 1.0 / sqrt(1.0 + t * t), sn = cs * t;
             const double2 ph = mk(gm.x / g, -gm.y / g);
-            if (l < nrows) {
-              const double2 aqt = cmul(aq, ph);
-              A[p * kAaaMax + l] = mk(cs * ap.x - sn * aqt.x, cs * ap.y - sn * aqt.y);
-              A[q * kAaaMax + l] = mk(sn * ap.x + cs * aqt.x, sn * ap.y + cs * aqt.y);
+#pragma unroll
+            for (int h = 0; h < H; ++h) {
+              const double2 aqt = cmul(aq[h], ph);
+              if (l + kGrp * h < nrows)
+                A[q * M + l + kGrp * h] =
+                    mk(sn * ap[h].x + cs * aqt.x, sn * ap[h].y + cs * aqt.y);
+              ap[h] = mk(cs * ap[h].x - sn * aqt.x, cs * ap[h].y - sn * aqt.y);
             }
             if (l < m) {
-              const double2 vp = V[p * kVs + l], vqt = cmul(V[q * kVs + l], ph);
-              V[p * kVs + l] = mk(cs * vp.x - sn * vqt.x, cs * vp.y - sn * vqt.y);
-              V[q * kVs + l] = mk(sn * vp.x + cs * vqt.x, sn * vp.y + cs * vqt.y);
+              const double2 vqt = cmul(V[q * mcap + l], ph);
+              V[q * mcap + l] = mk(sn * vp.x + cs * vqt.x, sn * vp.y + cs * vqt.y);
+              vp = mk(cs * vp.x - sn * vqt.x, cs * vp.y - sn * vqt.y);
             }
+            al = norm2(ap);
           }
+          if (turned) {
+#pragma unroll
+            for (int h = 0; h < H; ++h)
+              if (l + kGrp * h < nrows) A[p * M + l + kGrp * h] = ap[h];
+            if (l < m) V[p * mcap + l] = vp;
+          }
+        }
         if (rot == 0) break;
       }
       // the right singular vector of the smallest singular value
       double smin = INFINITY;
       for (int c = 0; c < m; ++c) {
-        const double2 a = l < nrows ? A[c * kAaaMax + l] : mk(0.0, 0.0);
-        const double s = wsum(cabs2a(a));
+        double2 a[H];
+        column(c, a);
+        const double s = norm2(a);
         if (s <= smin) {  // the last of equal ones, as ZGESDD's descending order
           smin = s;
           cmin = c;
@@ -198,31 +268,35 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
       }
     }
     __syncwarp();
-    if (l < m) wgt[l] = V[cmin * kVs + l];
+    if (l < m) wgt[l] = V[cmin * mcap + l];
     __syncwarp();
     // update_fit (:228-258)
-    if (pt && !sup) {
-      double2 num = mk(0.0, 0.0), den = mk(0.0, 0.0);
-      for (int c = 0; c < m; ++c) {
-        const double2 cc = cauchy(zl, pos[c]);
-        num = cadd(num, cmul(cc, cmul(wgt[c], val[c])));
-        den = cadd(den, cmul(cc, wgt[c]));
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+      if (pt[h] && !sup[h]) {
+        double2 num = zero, den = zero;
+        for (int c = 0; c < m; ++c) {
+          const double2 cc = cauchy(zl[h], pos[c]);
+          num = cadd(num, cmul(cc, cmul(wgt[c], val[c])));
+          den = cadd(den, cmul(cc, wgt[c]));
+        }
+        fit[h] = cdiv(num, den);
       }
-      fit = cdiv(num, den);
-    }
     // converged (:276-282) or max_step_reached (:285-292)
-    const double err = wmax(pt ? (cabsa(csub(fit, fl)) <= thres_abs ? 0.0 : 1.0) : 0.0);
-    if (err == 0.0 || m >= mp) break;
+#pragma unroll
+    for (int h = 0; h < H; ++h)
+      d[h] = pt[h] ? (cabsa(csub(fit[h], fl[h])) <= thres_abs ? 0.0 : 1.0) : 0.0;
+    if (wmax<H>(d) == 0.0 || m >= mp) break;
   }
   __syncwarp();
   if (m > mcap) {  // flagged: the coefficients are left as NaN
-    for (int s = l; s < M; s += 64) w[(int64_t)s * ne + e] = mk(NAN, NAN);
+    for (int s = l; s < M; s += kGrp) w[(int64_t)s * ne + e] = mk(NAN, NAN);
     return;
   }
   if (model == 4) {
     const int mmax = max_point;
-    for (int s = l; s < M; s += 64) {
-      double2 v = mk(0.0, 0.0);
+    for (int s = l; s < M; s += kGrp) {
+      double2 v = zero;
       if (s < m) v = pos[s];
       else if (s >= mmax && s < mmax + m) v = val[s - mmax];
       else if (s >= 2 * mmax && s < 2 * mmax + m) v = wgt[s - 2 * mmax];
@@ -233,9 +307,10 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
   // model 5: poles (zeros of the denominator) by Aberth-Ehrlich, then the
   // residues of calculate_residual (:458-500) and pole_correction's filter
   const int nr = m - 1;
-  double2 cen = wsum2(l < m ? pos[l] : mk(0.0, 0.0));
+  const double2 mine[1] = {l < m ? pos[l] : zero};
+  double2 cen = wsum2<1>(mine);
   cen = mk(cen.x / m, cen.y / m);
-  double rad = wmax(l < m ? cabsa(csub(pos[l], cen)) : 0.0);
+  double rad = lanes::max<kGrp>(l < m ? cabsa(csub(pos[l], cen)) : 0.0);
   if (!(rad > 0.0)) rad = 1.0;
   double2 lk = mk(0.0, 0.0);
   if (l < nr) {
@@ -247,7 +322,7 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
   double prev = INFINITY;
   for (int it = 0; it < kAberthIters; ++it) {
     __syncwarp();
-    lam[l] = lk;
+    if (l < nr) lam[l] = lk;
     __syncwarp();
     if (!done) {
       double2 sd = mk(0.0, 0.0), sd1 = mk(0.0, 0.0), sq = mk(0.0, 0.0);
@@ -272,7 +347,7 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
       done = a <= 1e-14 * al || (a >= prev && a <= 1e-10 * al);
       prev = a;
     }
-    if (__ballot(!done) == 0ull) break;
+    if (gballot(!done) == 0u) break;
   }
   // finite zeros only (the pencil's infinite eigenvalues are not zeros of
   // the denominator; a zero run off to infinity means sum w_j = 0)
@@ -286,21 +361,21 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
     res = mk(res.x / 4.0, res.y / 4.0);
   }
   const bool keep = finite_pole && cabsa(res) > thres;
-  const uint64_t kmask = __ballot(keep);
-  const int cnt = __popcll(kmask), half = M / 2;
+  const uint32_t kmask = gballot(keep);
+  const int cnt = __popc(kmask), half = M / 2;
   if (cnt > half) {
     if (l == 0) status[1] = 1;
-    for (int s = l; s < M; s += 64) w[(int64_t)s * ne + e] = mk(NAN, NAN);
+    for (int s = l; s < M; s += kGrp) w[(int64_t)s * ne + e] = mk(NAN, NAN);
     return;
   }
   __syncwarp();
   if (keep) {
-    const int k = __popcll(kmask & below(l));
+    const int k = __popc(kmask & (uint32_t)below(l));
     pos[k] = lk;   // the support points are no longer needed
     val[k] = res;
   }
   __syncwarp();
-  for (int s = l; s < M; s += 64) {
+  for (int s = l; s < M; s += kGrp) {
     double2 v = mk(0.0, 0.0);
     if (s < cnt) v = pos[s];
     else if (s >= half && s < half + cnt) v = val[s - half];
@@ -325,11 +400,15 @@ void aaa_coeffs(int model, double thres, int64_t ne, int nfreq, const double2 *z
   // unique)
   const int max_point = model == 4 ? nfreq / 3 : nfreq;
   const int mcap = model == 4 ? nfreq / 3 : nfreq / 2;
-  const size_t lds = sizeof(double2) * (size_t)aaa_lds(mcap);
+  const size_t lds = 2 * sizeof(double2) * (size_t)aaa_lds(nfreq, mcap);  // <= 102400
   DevBuf<int32_t> status(2);
   SGW_HIP(hipMemsetAsync(status.p, 0, 2 * sizeof(int32_t), st));
-  k_aaa_coeffs<<<(unsigned)ne, 64, lds, st>>>(ne, nfreq, mesh, thres, model, max_point, mcap,
-                                              d_w, status.p);
+  auto *kern = nfreq <= kGrp ? k_aaa_coeffs<1> : k_aaa_coeffs<2>;
+  if (lds > 64 * 1024)
+    SGW_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  kern<<<(unsigned)((ne + 1) / 2), 64, lds, st>>>(ne, nfreq, mesh, thres, model, max_point, mcap,
+                                                  d_w, status.p);
   SGW_HIP(hipGetLastError());
   int32_t h[2] = {0, 0};
   SGW_HIP(hipMemcpyAsync(h, status.p, sizeof(h), hipMemcpyDeviceToHost, st));
