@@ -8,14 +8,14 @@
 // same frequency sum is one long-K GEMM per output frequency:
 //   Sigma[i] = alpha [w_0 G[i][0] | ... | w_{nin-1} G[i][nin-1]] x [W[0]; ...; W[nin-1]].
 //
-// Kernel: one 128 x 64 complex tile of Sigma[i] per block, four waves of
-// 64 x 32; K staged through LDS 16 at a time; each complex 16 x 16 x 4 step
-// is four real v_mfma_f64_16x16x4f64 (re*re - im*im, re*im + im*re) into
-// FP64 accumulators.
+// Kernel: one complex tile of Sigma[i] per block of four waves, K staged through
+// LDS; each complex 16 x 16 x 4 step is four real v_mfma_f64_16x16x4f64
+// (re*re - im*im, re*im + im*re) into FP64 accumulators.
 #include "sgw.h"
 
 #include <cmath>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "ktimer.h"
@@ -26,7 +26,7 @@ namespace {
 
 typedef double v4d __attribute__((ext_vector_type(4)));
 
-constexpr int kSBM = 128, kSBN = 64, kSBK = 16, kSPad = 1;
+constexpr int kSBM = 128, kSBN = 64, kSBK = 16, kSPad = 1;  // FP32 split kernel
 
 struct SigmaArgs {
   int n;
@@ -49,89 +49,122 @@ __device__ inline int xcd_tile(int b, int nblocks) {
   return (b % 8) * per + b / 8;
 }
 
-__global__ __launch_bounds__(256) void k_sigma_f64(SigmaArgs a) {
-  __shared__ double2 As[kSBK][kSBM + kSPad];
-  __shared__ double2 Bs[kSBK][kSBN + kSPad];
+// BM x BN = 32 TM x 32 TN complex tile of Sigma[i] per block, four waves of
+// 16 TM x 16 TN.  K is staged kBK at a time through two LDS buffers: a stage's
+// values are fetched into registers while the previous one multiplies and go
+// to the other buffer after it, one barrier a stage.  The products of an
+// accumulator are spread over the wave's tile, so that none waits for the one
+// before it.
+constexpr int kBK = 8;
+
+template <int TM, int TN>
+__global__ __launch_bounds__(256, TM * TN > 2 ? 3 : 4) void k_sigma_f64(SigmaArgs a) {
+  constexpr int BM = 32 * TM, BN = 32 * TN, NA = BM * kBK / 256, NB = BN * kBK / 256;
+  __shared__ double2 As[2][kBK][BM + kSPad];
+  __shared__ double2 Bs[2][kBK][BN + kSPad];
   const int t = xcd_tile(blockIdx.x, a.nblocks);
   const int tiles = a.tiles_m * a.tiles_n;
   if (t >= tiles * a.nout) return;
   const int i = t / tiles, tt = t % tiles;
-  const int m0 = (tt % a.tiles_m) * kSBM, n0 = (tt / a.tiles_m) * kSBN;
+  const int m0 = (tt % a.tiles_m) * BM, n0 = (tt / a.tiles_m) * BN;
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int wm = (wv & 1) * 64, wn = (wv >> 1) * 32;
+  const int wm = (wv & 1) * 16 * TM, wn = (wv >> 1) * 16 * TN;
   const int lr = lane & 15, lk = lane >> 4;
   const int n = a.n;
   const int64_t ld = a.ld;
-  v4d cre[4][2], cim[4][2];
+  v4d cre[TM][TN], cim[TM][TN];
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
+  for (int r = 0; r < TM; ++r)
 #pragma unroll
-    for (int c = 0; c < 2; ++c) {
+    for (int c = 0; c < TN; ++c) {
       cre[r][c] = v4d{0, 0, 0, 0};
       cim[r][c] = v4d{0, 0, 0, 0};
     }
-  const int arow = tid & 127, ak = tid >> 7;  // A staging: 8 (row, k) per thread
-  const int bk = tid & 15, bc = tid >> 4;     // B staging: 4 (k, col) per thread
   // stages t = (j, kk): K runs over the G'' index of every convolution
-  // frequency in turn; the next stage's tiles are fetched into registers
-  // while the MFMAs of the current one run
-  const int nk = (n + kSBK - 1) / kSBK, nstage = a.nin * nk;
-  double2 ra[8], rb[4];
+  // frequency in turn
+  const int nk = (n + kBK - 1) / kBK, nstage = a.nin * nk;
+  double2 ra[NA], rb[NB];
   double rw = 0;
-  auto fetch = [&](int t) {
-    const int j = t / nk, kk = (t % nk) * kSBK;
-    const double2 *Gij = a.G + (int64_t)i * a.gsi + (int64_t)j * a.gsj;
-    const double2 *Wj = a.W + (int64_t)j * a.wsj;
-    rw = a.wt[j];
+  int fj = 0, fk = 0;  // frequency and first G'' of the next fetch
+  auto fetch = [&] {
+    const double2 *Gij = a.G + (int64_t)i * a.gsi + (int64_t)fj * a.gsj;
+    const double2 *Wj = a.W + (int64_t)fj * a.wsj;
+    rw = a.wt[fj];
 #pragma unroll
-    for (int r = 0; r < 8; ++r) {
-      const int gm = m0 + arow, gk = kk + ak + 2 * r;
+    for (int r = 0; r < NA; ++r) {
+      const int e = tid + 256 * r, gm = m0 + e % BM, gk = fk + e / BM;
       ra[r] = (gm < n && gk < n) ? Gij[gm + (int64_t)gk * ld] : mk(0, 0);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int gk = kk + bk, gn = n0 + bc + 16 * r;
+    for (int r = 0; r < NB; ++r) {
+      const int e = tid + 256 * r, gk = fk + e % kBK, gn = n0 + e / kBK;
       rb[r] = (gk < n && gn < n) ? Wj[gk + (int64_t)gn * ld] : mk(0, 0);
     }
-  };
-  fetch(0);
-  for (int t = 0; t < nstage; ++t) {
-    {
-      __syncthreads();
-#pragma unroll
-      for (int r = 0; r < 8; ++r) As[ak + 2 * r][arow] = mk(ra[r].x * rw, ra[r].y * rw);
-#pragma unroll
-      for (int r = 0; r < 4; ++r) Bs[bk][bc + 16 * r] = rb[r];
-      __syncthreads();
-      if (t + 1 < nstage) fetch(t + 1);
-#pragma unroll
-      for (int k4 = 0; k4 < kSBK / 4; ++k4) {
-        const int kr = 4 * k4 + lk;
-        double2 av[4], bv[2];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) av[r] = As[kr][wm + 16 * r + lr];
-#pragma unroll
-        for (int c = 0; c < 2; ++c) bv[c] = Bs[kr][wn + 16 * c + lr];
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int c = 0; c < 2; ++c) {
-            cre[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[r].x, bv[c].x, cre[r][c], 0, 0, 0);
-            cre[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(-av[r].y, bv[c].y, cre[r][c], 0, 0, 0);
-            cim[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[r].x, bv[c].y, cim[r][c], 0, 0, 0);
-            cim[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[r].y, bv[c].x, cim[r][c], 0, 0, 0);
-          }
-      }
+    fk += kBK;
+    if (fk >= n) {
+      fk = 0;
+      ++fj;
     }
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int r = 0; r < NA; ++r) {
+      const int e = tid + 256 * r;
+      As[buf][e / BM][e % BM] = mk(ra[r].x * rw, ra[r].y * rw);
+    }
+#pragma unroll
+    for (int r = 0; r < NB; ++r) {
+      const int e = tid + 256 * r;
+      Bs[buf][e % kBK][e / kBK] = rb[r];
+    }
+  };
+  fetch();
+  store(0);
+  __syncthreads();
+  for (int t = 0; t < nstage; ++t) {
+    const int buf = t & 1;
+    const bool more = t + 1 < nstage;
+    if (more) fetch();
+#pragma unroll
+    for (int k4 = 0; k4 < kBK / 4; ++k4) {
+      const int kr = 4 * k4 + lk;
+      double2 av[TM], bv[TN];
+#pragma unroll
+      for (int r = 0; r < TM; ++r) av[r] = As[buf][kr][wm + 16 * r + lr];
+#pragma unroll
+      for (int c = 0; c < TN; ++c) bv[c] = Bs[buf][kr][wn + 16 * c + lr];
+#pragma unroll
+      for (int r = 0; r < TM; ++r)
+#pragma unroll
+        for (int c = 0; c < TN; ++c)
+          cre[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[r].x, bv[c].x, cre[r][c], 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < TM; ++r)
+#pragma unroll
+        for (int c = 0; c < TN; ++c)
+          cim[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[r].x, bv[c].y, cim[r][c], 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < TM; ++r)
+#pragma unroll
+        for (int c = 0; c < TN; ++c)
+          cre[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(-av[r].y, bv[c].y, cre[r][c], 0, 0, 0);
+#pragma unroll
+      for (int r = 0; r < TM; ++r)
+#pragma unroll
+        for (int c = 0; c < TN; ++c)
+          cim[r][c] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[r].y, bv[c].x, cim[r][c], 0, 0, 0);
+    }
+    if (more) store(buf ^ 1);
+    __syncthreads();
   }
   // v_mfma_f64_16x16x4f64 leaves D(lane / 16 + 4 q, lane % 16) in element q
   // of a lane's accumulator (A(lane % 16, lane / 16), B(lane / 16, lane % 16)
   // in its operands); checked on the device
   double2 *Si = a.S + (int64_t)i * a.ssi;
 #pragma unroll
-  for (int r = 0; r < 4; ++r)
+  for (int r = 0; r < TM; ++r)
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
+    for (int c = 0; c < TN; ++c)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int row = m0 + wm + 16 * r + lk + 4 * q, col = n0 + wn + 16 * c + lr;
@@ -143,6 +176,127 @@ __global__ __launch_bounds__(256) void k_sigma_f64(SigmaArgs a) {
           *p = v;
         }
       }
+}
+
+// Small outputs: one 16 x 16 tile per block, its four waves taking every fourth
+// K chunk straight from memory to the matrix registers, the next chunk in
+// flight; their sums meet in LDS.  Four times the blocks of a 32 x 32 tile
+// and no barrier in the K loop.
+__global__ __launch_bounds__(256, 2) void k_sigma_f64_small(SigmaArgs a) {
+  constexpr int KC = 16, ST = KC / 4;
+  __shared__ double red[3][64][9];
+  const int t = xcd_tile(blockIdx.x, a.nblocks);
+  const int tiles = a.tiles_m * a.tiles_n;
+  if (t >= tiles * a.nout) return;
+  const int i = t / tiles, tt = t % tiles;
+  const int m0 = (tt % a.tiles_m) * 16, n0 = (tt / a.tiles_m) * 16;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+  const int n = a.n;
+  const int64_t ld = a.ld;
+  const bool am = m0 + lr < n, bn = n0 + lr < n;
+  v4d cre{0, 0, 0, 0}, cim{0, 0, 0, 0};
+  double2 av[ST], bv[ST];
+  double rw = 0;
+  int fj = 0, fk = wv * KC;  // frequency and first G'' of the next chunk
+  auto settle = [&] {
+    while (fk >= n && fj < a.nin) {  // chunks go round the waves within a frequency
+      fk = wv * KC;
+      ++fj;
+      if (fk >= n) fk = n;           // fewer chunks than waves: this one has none
+    }
+  };
+  auto fetch = [&] {
+    const double2 *Gij = a.G + (int64_t)i * a.gsi + (int64_t)fj * a.gsj + m0 + lr;
+    const double2 *Wj = a.W + (int64_t)fj * a.wsj + (int64_t)(n0 + lr) * ld;
+    rw = a.wt[fj];
+#pragma unroll
+    for (int s = 0; s < ST; ++s) {
+      const int k = fk + 4 * s + lk;
+      av[s] = am && k < n ? Gij[(int64_t)k * ld] : mk(0, 0);
+      bv[s] = bn && k < n ? Wj[k] : mk(0, 0);
+    }
+    fk += 4 * KC;
+    settle();
+  };
+  settle();
+  bool more = fj < a.nin;
+  if (more) fetch();
+  while (more) {
+    double2 ac[ST], bc[ST];
+#pragma unroll
+    for (int s = 0; s < ST; ++s) {
+      ac[s] = mk(av[s].x * rw, av[s].y * rw);
+      bc[s] = bv[s];
+    }
+    more = fj < a.nin;
+    if (more) fetch();
+#pragma unroll
+    for (int s = 0; s < ST; ++s) {
+      cre = __builtin_amdgcn_mfma_f64_16x16x4f64(ac[s].x, bc[s].x, cre, 0, 0, 0);
+      cim = __builtin_amdgcn_mfma_f64_16x16x4f64(ac[s].x, bc[s].y, cim, 0, 0, 0);
+      cre = __builtin_amdgcn_mfma_f64_16x16x4f64(-ac[s].y, bc[s].y, cre, 0, 0, 0);
+      cim = __builtin_amdgcn_mfma_f64_16x16x4f64(ac[s].y, bc[s].x, cim, 0, 0, 0);
+    }
+  }
+  if (wv) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      red[wv - 1][lane][q] = cre[q];
+      red[wv - 1][lane][4 + q] = cim[q];
+    }
+  }
+  __syncthreads();
+  if (wv) return;
+  double2 *Si = a.S + (int64_t)i * a.ssi;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const int row = m0 + lk + 4 * q, col = n0 + lr;
+    double2 acc = mk(cre[q], cim[q]);
+    for (int w = 0; w < 3; ++w) acc = cadd(acc, mk(red[w][lane][q], red[w][lane][4 + q]));
+    if (row < n && col < n) {
+      double2 v = cmul(a.alpha, acc);
+      double2 *p = Si + row + (int64_t)col * ld;
+      if (a.accumulate) v = cadd(*p, v);
+      *p = v;
+    }
+  }
+}
+
+// FP64 tiles: 16-tiles of a wave (TM x TN; 0: the 16 x 16 kernel) and the time of
+// one unit of work (a 32 x 32 tile over K) on a full CU, relative to the
+// largest tile's: staging and operand reads weigh more on a small tile.
+// Measured at n = 1500, 8 outputs: 62.2, 53.1, 49.0 and 33 TFLOP/s (128 x 64
+// and 96 x 64 tiles, two waves to a SIMD: 60.4 and 59.1, and fuller CUs never
+// need them).
+struct Tile {
+  int tm, tn;
+  double unit;
+};
+constexpr Tile kTiles[] = {{2, 2, 1.0}, {2, 1, 1.17}, {1, 1, 1.3}, {0, 0, 1.35}};
+constexpr double kSmallPerN = 0.2 / 1500;  // the 16 x 16 kernel's operands outgrow the caches with n
+int tile_edge(int t) { return t ? 32 * t : 16; }
+
+// The tile that leaves the fullest CU the least work: the blocks of a CU share
+// its matrix cores, so its time is the sum over them, and a CU with few
+// blocks hides less of their latency.  One tile size for all (128 x 64 before)
+// left most CUs idle at small n; measured before and after: n = 1500, 4 outputs,
+// 8 frequencies 18.6 -> 14.0 ms; 700, 1, 8: 1737 -> 511 us; 300, 2, 8: 752 ->
+// 95 us; 150, 1, 8: 395 -> 27 us.
+Tile pick_tile(int n, int nout) {
+  Tile best = kTiles[0];
+  double least = INFINITY;
+  for (const Tile &t : kTiles) {
+    const int bm = tile_edge(t.tm), bn = tile_edge(t.tn);
+    const int64_t blocks = (int64_t)((n + bm - 1) / bm) * ((n + bn - 1) / bn) * nout;
+    const double rounds = (double)((blocks + 255) / 256);
+    const double unit = t.unit + (t.tm ? 0.0 : kSmallPerN * n);
+    const double cost = rounds * (bm * bn / 1024.0) * unit * (1.0 + 0.4 / (rounds * std::sqrt(rounds)));
+    if (cost < least) {
+      least = cost;
+      best = t;
+    }
+  }
+  return best;
 }
 
 // ---------------------------------------------------------------------------
@@ -363,20 +517,30 @@ int sgw_sigma_conv_device(const sgw_sigma_conv_desc *desc, const sgw_complex *d_
     a.alpha = make_double2(alpha.re, alpha.im);
     a.S = reinterpret_cast<double2 *>(d_sigma);
     a.accumulate = c.accumulate ? 1 : 0;
-    a.tiles_m = (c.n + sgw::kSBM - 1) / sgw::kSBM;
-    a.tiles_n = (c.n + sgw::kSBN - 1) / sgw::kSBN;
+    const bool fp64 = c.precision == SGW_SIGMA_FP64;
+    const sgw::Tile tile = sgw::pick_tile(c.n, c.nout);
+    const int bm = fp64 ? sgw::tile_edge(tile.tm) : sgw::kSBM;
+    const int bn = fp64 ? sgw::tile_edge(tile.tn) : sgw::kSBN;
+    a.tiles_m = (c.n + bm - 1) / bm;
+    a.tiles_n = (c.n + bn - 1) / bn;
     const int64_t blocks = (int64_t)a.tiles_m * a.tiles_n * c.nout;
     SGW_REQUIRE(blocks < (1ll << 31) - 8, SGW_E_SHAPE, "sigma_conv: too many tiles");
     a.nblocks = (int)(((blocks + 7) / 8) * 8);
     hipStream_t st = (hipStream_t)stream;
-    {
-      if (c.precision == SGW_SIGMA_FP64) {
-        sgw::KScope ks("sigma_f64", st);
-        sgw::k_sigma_f64<<<a.nblocks, 256, 0, st>>>(a);
-      } else {
-        sgw::KScope ks("sigma_f32s", st);
-        sgw::k_sigma_f32s<<<a.nblocks, 256, 0, st>>>(a);
-      }
+    if (fp64) {
+      sgw::KScope ks("sigma_f64", st);
+      auto go = [&](auto tm, auto tn) {
+        if (tile.tm == decltype(tm)::value && tile.tn == decltype(tn)::value)
+          sgw::k_sigma_f64<decltype(tm)::value, decltype(tn)::value><<<a.nblocks, 256, 0, st>>>(a);
+      };
+      using std::integral_constant;
+      go(integral_constant<int, 2>{}, integral_constant<int, 2>{});
+      go(integral_constant<int, 2>{}, integral_constant<int, 1>{});
+      go(integral_constant<int, 1>{}, integral_constant<int, 1>{});
+      if (tile.tm == 0) sgw::k_sigma_f64_small<<<a.nblocks, 256, 0, st>>>(a);
+    } else {
+      sgw::KScope ks("sigma_f32s", st);
+      sgw::k_sigma_f32s<<<a.nblocks, 256, 0, st>>>(a);
     }
     SGW_HIP(hipGetLastError());
     return 0;

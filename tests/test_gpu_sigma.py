@@ -128,3 +128,25 @@ def test_conv_fp32_split_matches_oracle(n, ld, nout, nin):
     print("fp32 split relative errors", errs, flush=True)
     assert max(errs) <= 2e-5
     assert min(errs) > 1e-12
+
+
+@pytest.mark.parametrize("n,nout,nin", [
+    (15, 1, 1), (16, 2, 3), (33, 1, 2),          # 16 x 16 tiles, K split over four waves
+    (449, 3, 2), (512, 2, 1),                    # 32 x 32
+    (703, 2, 1),                                 # 64 x 32
+    (1025, 1, 1), (769, 4, 1)])                  # 64 x 64
+def test_conv_tiles(n, nout, nin):
+    """The FP64 kernel's tile sizes at their edges, against the same sum in
+    numpy: K = nin n products each way, as above."""
+    print(f"sigma_conv tiles n={n} nout={nout} nin={nin}", flush=True)
+    rng = np.random.Generator(np.random.PCG64(n))
+    G, W = _rand(rng, nout, nin, n, n), _rand(rng, nin, n, n)
+    wt = rng.uniform(0.1, 1.0, nin)
+    alpha = complex(0.7, -0.2)
+    ref = alpha * np.einsum("j,ijab->iab", wt, np.matmul(G, W[None]))
+    d_s = _to_dev_colmajor(np.zeros_like(ref), n)
+    sigma.conv_device(_to_dev_colmajor(G, n), _to_dev_colmajor(W, n), torch.from_numpy(wt).to(DEV),
+                      d_s, n, n, nout, nin, alpha)
+    got = _from_dev_colmajor(d_s, n)
+    for i in range(nout):
+        assert np.linalg.norm(got[i] - ref[i]) <= FP64_TOL * np.linalg.norm(ref[i]), i
