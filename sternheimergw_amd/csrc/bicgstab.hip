@@ -18,79 +18,82 @@
 #include "sgw_internal.h"
 #include "bicgstab.h"
 #include "ktimer.h"
+#include "lanes.h"
 #include "operators.h"
 
 #include <algorithm>
 #include <cmath>
 #include <cstdlib>
+#include <type_traits>
 
 namespace sgw {
 
 namespace {
 
 constexpr int kBlock = 256;
-// slots from which a BiCG seed half step runs as one launch (one block per
-// system) rather than two (dot product, then the update over a grid of
-// tiles): the one-launch form is faster at 1024 slots, slower at 256
-constexpr int kFuseHalves = 512;
 constexpr int kShiftGroups = 4;  // default shifted-system groups per k_shift_cycle block
 
 // ---------------------------------------------------------------------------
 // reductions
 // ---------------------------------------------------------------------------
-__device__ inline double2 wave_sum(double2 v) {
-  for (int off = 32; off > 0; off >>= 1) {
-    v.x += __shfl_xor(v.x, off, 64);
-    v.y += __shfl_xor(v.y, off, 64);
-  }
-  return v;
+// Blocks that hold one system sum over its vector with 256 threads, in the same
+// order whatever the batch, and run the element-wise updates that follow on
+// all of theirs: long vectors take 1024, which keeps enough loads in flight
+// where few systems run; short ones gain nothing from more waves.
+constexpr int kSumThreads = 256;
+template <typename F> void with_threads(int64_t ld, F &&f) {
+  if (ld <= 512) f(std::integral_constant<int, 256>{});
+  else f(std::integral_constant<int, 1024>{});
 }
 
-// Block-wide sum (deterministic); every thread returns the total.
-template <int NT> __device__ inline double2 block_sum(double2 v, double2 *lds) {
-  v = wave_sum(v);
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  __syncthreads();
-  if (lane == 0) lds[wid] = v;
-  __syncthreads();
-  double2 t = mk(0, 0);
-  if (threadIdx.x < 64) {
-    t = threadIdx.x < NT / 64 ? lds[threadIdx.x] : mk(0, 0);
-    t = wave_sum(t);
-    if (threadIdx.x == 0) lds[0] = t;
+// Sums over a block of K values from each of NV 64-value vectors per wavefront
+// (vector m of wave w is number w + m waves): a butterfly within each, then
+// one over the vectors; every thread returns the totals.  One barrier:
+// successive calls alternate between the halves of lds.
+template <int NW, int NV, int K> struct BlockSum {
+  double lds[2][NW * NV][K];
+  __device__ void run(double (&v)[NV][K], double (&out)[K], int &turn) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    double(&buf)[NW * NV][K] = lds[turn & 1];
+    ++turn;
+    if (wid < NW) {
+#pragma unroll
+      for (int m = 0; m < NV; ++m)
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          const double t = lanes::sum<64>(v[m][k]);
+          if (lane == 0) buf[wid + m * NW][k] = t;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      double t[NW * NV];
+#pragma unroll
+      for (int w = 0; w < NW * NV; ++w) t[w] = buf[w][k];
+#pragma unroll
+      for (int o = NW * NV / 2; o > 0; o >>= 1)
+#pragma unroll
+        for (int w = 0; w < o; ++w) t[w] += t[w + o];
+      out[k] = t[0];
+    }
   }
-  __syncthreads();
-  t = lds[0];
-  return t;
-}
+};
 
-// sum_i a[i] * b[i]  (ZDOTU) over n entries by one kBlock block; every thread
-// returns the total
+// sum_i a[i] * b[i]  (ZDOTU) over n entries by the first 256 threads of a block;
+// every thread returns the total
+using DotSum = BlockSum<kSumThreads / 64, 1, 2>;
 __device__ inline double2 block_dotu(const double2 *__restrict__ pa,
-                                     const double2 *__restrict__ pb, int64_t n, double2 *lds) {
+                                     const double2 *__restrict__ pb, int64_t n, DotSum &bs,
+                                     int &turn) {
   double2 acc = mk(0, 0);
+  if (threadIdx.x < kSumThreads) {
 #pragma unroll 8
-  for (int64_t i = threadIdx.x; i < n; i += kBlock) cmac(acc, pa[i], pb[i]);  // loads in flight
-  return block_sum<kBlock>(acc, lds);
-}
-
-// out[s] = sqrt(sum_i |a[s][i]|^2)
-__global__ __launch_bounds__(kBlock) void k_norm(int nsys, const int32_t *__restrict__ active,
-                                                 const double2 *__restrict__ a, int64_t sa,
-                                                 int64_t n, double *__restrict__ out) {
-  __shared__ double2 lds[kBlock / 64];
-  const int s = blockIdx.x;
-  if (!active[s]) return;
-  const double2 *pa = a + s * sa;
-  double2 acc = mk(0, 0);
-#pragma unroll 8
-  for (int64_t i = threadIdx.x; i < n; i += kBlock) {
-    double2 v = pa[i];
-    acc.x = fma(v.x, v.x, acc.x);
-    acc.x = fma(v.y, v.y, acc.x);
+    for (int64_t i = threadIdx.x; i < n; i += kSumThreads) cmac(acc, pa[i], pb[i]);  // in flight
   }
-  acc = block_sum<kBlock>(acc, lds);
-  if (threadIdx.x == 0) out[s] = sqrt(acc.x);
+  double v[1][2] = {{acc.x, acc.y}}, t[2];
+  bs.run(v, t, turn);
+  return mk(t[0], t[1]);
 }
 
 // ---------------------------------------------------------------------------
@@ -137,23 +140,6 @@ __device__ inline void bicg_s1_body(int s, int begin, int commit, Scal sc,
   sc.rho_old[s] = rho;
 }
 
-// rho = (r_j, r0~) by block s, then the scalar step above by its thread 0
-__global__ __launch_bounds__(kBlock) void k_dotu_s1(const int32_t *__restrict__ active,
-                                                    const double2 *__restrict__ a, int64_t sa,
-                                                    const double2 *__restrict__ b, int64_t n,
-                                                    int begin, int commit, Scal sc,
-                                                    int32_t *__restrict__ fresh,
-                                                    int32_t *__restrict__ count) {
-  __shared__ double2 lds[kBlock / 64];
-  const int s = blockIdx.x;
-  if (!active[s]) return;
-  const double2 acc = block_dotu(a + s * sa, b + s * n, n, lds);
-  if (threadIdx.x == 0) {
-    sc.dot[s] = acc;
-    bicg_s1_body(s, begin, commit, sc, fresh, count, acc);
-  }
-}
-
 // bicgstab.f90:614-670  alpha = rho / (u_{j+1}, r0~) and the shifted scalars
 // of shifted system k; `dot` = (u_{j+1}, r0~).  The per-step factors go to slot
 // (s*nsh + k)*l + j: the shifted vectors are updated once per iteration, for
@@ -184,20 +170,6 @@ __device__ inline void bicg_s2_body(int s, int k, int nsh, int l, int j, Scal sc
   sc.ia[pj] = cdiv(one, alpha_s);
 }
 
-// (u_{j+1}, r0~) by block s, then the shifted scalars of system s, one thread
-// per shifted system (the k = 0 thread also stores the seed alpha)
-__global__ __launch_bounds__(kBlock) void k_dotu_s2(const int32_t *__restrict__ active,
-                                                    const double2 *__restrict__ a, int64_t sa,
-                                                    const double2 *__restrict__ b, int64_t n,
-                                                    int nsh, int l, int j, Scal sc) {
-  __shared__ double2 lds[kBlock / 64];
-  const int s = blockIdx.x;
-  if (!active[s]) return;
-  const double2 acc = block_dotu(a + s * sa, b + s * n, n, lds);
-  if (threadIdx.x == 0) sc.dot[s] = acc;
-  for (int k = threadIdx.x; k < max(nsh, 1); k += kBlock) bicg_s2_body(s, k, nsh, l, j, sc, acc);
-}
-
 // ---------------------------------------------------------------------------
 // element-wise vector kernels; grid = (ceil(ld/kBlock), S)
 // ---------------------------------------------------------------------------
@@ -219,47 +191,6 @@ struct Vecs {
   __device__ double2 *sx(int s, int k) const { return SX + ((int64_t)s * nsh + k) * ld; }
 };
 
-// L7-L8: u_i = r_i - beta u_i, i = 0..j
-__global__ __launch_bounds__(kBlock) void k_bicg_v1(int j, const int32_t *__restrict__ active,
-                                                    Vecs v, Scal sc) {
-  const int s = blockIdx.y;
-  if (!active[s]) return;
-  const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (e >= v.ld) return;
-  const double2 mb = cneg(sc.beta[s]);
-  for (int i = 0; i <= j; ++i) {
-    double2 *pu = v.u(s, i) + e;
-    double2 t = cmul(mb, *pu);
-    *pu = cadd(t, v.r(s, i)[e]);
-  }
-}
-
-// Seed half of step j after the matrix-vector product: L21-L22 (seed
-// residuals r_i -= alpha u_{i+1}) and L25 (x += alpha u_0).  The residuals
-// r_0..r_j before the update are kept as snapshots for the shifted systems
-// (their L15/L19 use them); after the last step, r_{l-1} after its update
-// (used by L26 of that step) is kept as well.
-__global__ __launch_bounds__(kBlock) void k_bicg_seed(int j, const int32_t *__restrict__ active,
-                                                      Vecs v, Scal sc) {
-  const int s = blockIdx.y;
-  if (!active[s]) return;
-  const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (e >= v.ld) return;
-  const double2 alpha = sc.alpha_new[s];
-  const double2 malpha = cneg(alpha);
-  for (int i = 0; i <= j; ++i) {
-    double2 t = v.r(s, i)[e];
-    v.rs(s, snap_index(j, i))[e] = t;
-    cmac(t, malpha, v.u(s, i + 1)[e]);
-    v.r(s, i)[e] = t;
-    if (j == v.l - 1 && i == j) v.rs(s, snap_final(v.l))[e] = t;
-  }
-  double2 *px = v.x(s) + e;
-  double2 t = *px;
-  cmac(t, alpha, v.u(s, 0)[e]);
-  *px = t;
-}
-
 // The seed halves of BiCG step j around its H-apply, one block per system
 // (bicgstab.f90:594-608, and 613-616 with 672-686; the shifted scalars
 // bicgstab.f90:617-670):
@@ -273,15 +204,17 @@ __global__ __launch_bounds__(kBlock) void k_bicg_seed(int j, const int32_t *__re
 //                 (x += alpha u_0).
 // A block reads its own system's vectors only, so the dot product and the
 // update that depends on it share one launch.
-__global__ __launch_bounds__(kBlock) void k_bicg_half1(int j, const int32_t *__restrict__ active,
-                                                       Vecs v, int begin, int commit, Scal sc,
-                                                       int32_t *__restrict__ fresh,
-                                                       int32_t *__restrict__ count) {
-  __shared__ double2 lds[kBlock / 64];
+template <int NT>
+__global__ __launch_bounds__(NT) void k_bicg_half1(int j, const int32_t *__restrict__ active,
+                                                   Vecs v, int begin, int commit, Scal sc,
+                                                   int32_t *__restrict__ fresh,
+                                                   int32_t *__restrict__ count) {
+  __shared__ DotSum bs;
   __shared__ double2 beta;
+  int turn = 0;
   const int s = blockIdx.x;
   if (!active[s]) return;
-  const double2 acc = block_dotu(v.r(s, j), v.RT + (int64_t)s * v.ld, v.ld, lds);
+  const double2 acc = block_dotu(v.r(s, j), v.RT + (int64_t)s * v.ld, v.ld, bs, turn);
   if (threadIdx.x == 0) {
     sc.dot[s] = acc;
     bicg_s1_body(s, begin, commit, sc, fresh, count, acc);
@@ -289,7 +222,7 @@ __global__ __launch_bounds__(kBlock) void k_bicg_half1(int j, const int32_t *__r
   }
   __syncthreads();
   const double2 mb = cneg(beta);
-  for (int64_t e = threadIdx.x; e < v.ld; e += kBlock)
+  for (int64_t e = threadIdx.x; e < v.ld; e += NT)
     for (int i = 0; i <= j; ++i) {
       double2 *pu = v.u(s, i) + e;
       double2 t = cmul(mb, *pu);
@@ -297,21 +230,19 @@ __global__ __launch_bounds__(kBlock) void k_bicg_half1(int j, const int32_t *__r
     }
 }
 
-__global__ __launch_bounds__(kBlock) void k_bicg_half2(int j, const int32_t *__restrict__ active,
-                                                       Vecs v, int nsh, int l, Scal sc) {
-  __shared__ double2 lds[kBlock / 64];
-  __shared__ double2 alpha_s;
+template <int NT>
+__global__ __launch_bounds__(NT) void k_bicg_half2(int j, const int32_t *__restrict__ active,
+                                                   Vecs v, int nsh, int l, Scal sc) {
+  __shared__ DotSum bs;
+  int turn = 0;
   const int s = blockIdx.x;
   if (!active[s]) return;
-  const double2 acc = block_dotu(v.u(s, j + 1), v.RT + (int64_t)s * v.ld, v.ld, lds);
-  if (threadIdx.x == 0) {
-    sc.dot[s] = acc;
-    alpha_s = cdiv(sc.rho[s], acc);  // the alpha bicg_s2_body stores as alpha_new
-  }
-  for (int k = threadIdx.x; k < max(nsh, 1); k += kBlock) bicg_s2_body(s, k, nsh, l, j, sc, acc);
-  __syncthreads();
-  const double2 alpha = alpha_s, malpha = cneg(alpha);
-  for (int64_t e = threadIdx.x; e < v.ld; e += kBlock) {
+  const double2 acc = block_dotu(v.u(s, j + 1), v.RT + (int64_t)s * v.ld, v.ld, bs, turn);
+  if (threadIdx.x == 0) sc.dot[s] = acc;
+  for (int k = threadIdx.x; k < max(nsh, 1); k += NT) bicg_s2_body(s, k, nsh, l, j, sc, acc);
+  // the alpha bicg_s2_body stores as alpha_new
+  const double2 alpha = cdiv(sc.rho[s], acc), malpha = cneg(alpha);
+  for (int64_t e = threadIdx.x; e < v.ld; e += NT) {
     for (int i = 0; i <= j; ++i) {
       double2 t = v.r(s, i)[e];
       v.rs(s, snap_index(j, i))[e] = t;
@@ -436,50 +367,16 @@ __global__ __launch_bounds__(kBlock) void k_mr_seed(const int32_t *__restrict__ 
 
 // Algorithm 4, MGS part and all scalars (one block per system).
 // bicgstab.f90:780-829 (seed) and :850-884 (per-shift Horner and gammas).
+struct MrLds {
+  double2 tau[(kMaxL + 1) * (kMaxL + 2) / 2];
+  double2 nu[kMaxL + 1];
+  double2 gam[kMaxL + 1], gp[kMaxL + 1], gpp[kMaxL + 1];
+};
+
+// the scalars from tau and gamma' in m (all threads, after a barrier)
 template <int NT>
-__global__ __launch_bounds__(NT) void k_mr_mgs(const int32_t *__restrict__ active, Vecs v, Scal sc,
-                                               int ntau, int nmu) {
-  const int s = blockIdx.x;
-  if (!active[s]) return;
-  __shared__ double2 lds[NT / 64];
-  __shared__ double2 tau[(kMaxL + 1) * (kMaxL + 2) / 2];
-  __shared__ double2 nu[kMaxL + 1];
-  __shared__ double2 gam[kMaxL + 1], gp[kMaxL + 1], gpp[kMaxL + 1];
-  const int l = v.l;
-  const int64_t ld = v.ld;
-  for (int jj = 1; jj <= l; ++jj) {
-    double2 *rj = v.r(s, jj);
-    int offset = jj * (jj + 1) / 2 + 1;
-    for (int ii = 1; ii <= jj - 1; ++ii) {
-      const double2 *ri = v.r(s, ii);
-      double2 acc = mk(0, 0);
-      for (int64_t e = threadIdx.x; e < ld; e += NT) cmac(acc, rj[e], ri[e]);
-      acc = block_sum<NT>(acc, lds);
-      double2 t = cdiv(acc, nu[ii]);
-      if (threadIdx.x == 0) tau[offset + ii - 1] = t;
-      const double2 mt = cneg(t);
-      for (int64_t e = threadIdx.x; e < ld; e += NT) {
-        double2 x = rj[e];
-        cmac(x, mt, ri[e]);
-        rj[e] = x;
-      }
-      __syncthreads();
-    }
-    double2 a1 = mk(0, 0), a2 = mk(0, 0);
-    const double2 *r0 = v.r(s, 0);
-    for (int64_t e = threadIdx.x; e < ld; e += NT) {
-      double2 x = rj[e];
-      cmac(a1, x, x);
-      cmac(a2, r0[e], x);
-    }
-    a1 = block_sum<NT>(a1, lds);
-    a2 = block_sum<NT>(a2, lds);
-    if (threadIdx.x == 0) {
-      nu[jj] = a1;
-      gp[jj] = cdiv(a2, a1);
-    }
-    __syncthreads();
-  }
+__device__ void mr_scalars(int s, int l, int nsh, int nmu, const Scal &sc, MrLds &m) {
+  double2 *tau = m.tau, *gam = m.gam, *gp = m.gp, *gpp = m.gpp;
   if (threadIdx.x == 0) {
     gam[l] = gp[l];                                                // L7
     sc.omega[s] = gam[l];
@@ -507,8 +404,8 @@ __global__ __launch_bounds__(NT) void k_mr_mgs(const int32_t *__restrict__ activ
   }
   __syncthreads();
   // per shift (one thread each): Horner (Algorithm 5), theta, gamma', gamma''
-  for (int k = threadIdx.x; k < v.nsh; k += NT) {
-    const int idx = s * v.nsh + k;
+  for (int k = threadIdx.x; k < nsh; k += NT) {
+    const int idx = s * nsh + k;
     const double2 sg = sc.sigma[idx], one = mk(1, 0);
     double2 g[kMaxL + 1];
     g[l] = cneg(gam[l]);
@@ -541,7 +438,130 @@ __global__ __launch_bounds__(NT) void k_mr_mgs(const int32_t *__restrict__ activ
     }
     cf[l] = cdiv(one, psi);                                        // L34 factor
   }
-  (void)ntau;
+}
+
+// Elements e = t + 1024 k of a thread's column are summed first, then 16
+// 64-element runs by butterflies, in both kernels.
+constexpr int kMrThreads = 1024;
+using MrSum = BlockSum<kMrThreads / 64, 1, 2>;
+__device__ inline double2 mr_sum(double2 a, MrSum &bs, int &turn) {
+  double v[1][2] = {{a.x, a.y}}, t[2];
+  bs.run(v, t, turn);
+  return mk(t[0], t[1]);
+}
+
+// Vectors longer than a block's registers hold, or l above 4
+__global__ __launch_bounds__(kMrThreads) void k_mr_mgs(const int32_t *__restrict__ active, Vecs v,
+                                                       Scal sc, int nmu) {
+  const int s = blockIdx.x;
+  if (!active[s]) return;
+  __shared__ MrSum bs;
+  __shared__ MrLds m;
+  int turn = 0;
+  const int l = v.l;
+  const int64_t ld = v.ld;
+  for (int jj = 1; jj <= l; ++jj) {
+    double2 *rj = v.r(s, jj);
+    int offset = jj * (jj + 1) / 2 + 1;
+    for (int ii = 1; ii <= jj - 1; ++ii) {
+      const double2 *ri = v.r(s, ii);
+      double2 acc = mk(0, 0);
+      for (int64_t e = threadIdx.x; e < ld; e += kMrThreads) cmac(acc, rj[e], ri[e]);
+      acc = mr_sum(acc, bs, turn);
+      double2 t = cdiv(acc, m.nu[ii]);
+      if (threadIdx.x == 0) m.tau[offset + ii - 1] = t;
+      const double2 mt = cneg(t);
+      for (int64_t e = threadIdx.x; e < ld; e += kMrThreads) {
+        double2 x = rj[e];
+        cmac(x, mt, ri[e]);
+        rj[e] = x;
+      }
+    }
+    double2 a1 = mk(0, 0), a2 = mk(0, 0);
+    const double2 *r0 = v.r(s, 0);
+    for (int64_t e = threadIdx.x; e < ld; e += kMrThreads) {
+      double2 x = rj[e];
+      cmac(a1, x, x);
+      cmac(a2, r0[e], x);
+    }
+    a1 = mr_sum(a1, bs, turn);
+    a2 = mr_sum(a2, bs, turn);
+    if (threadIdx.x == 0) {
+      m.nu[jj] = a1;
+      m.gp[jj] = cdiv(a2, a1);
+    }
+    __syncthreads();
+  }
+  mr_scalars<kMrThreads>(s, l, v.nsh, nmu, sc, m);
+}
+
+// The same with r_0..r_L in registers: every residual is read and written once,
+// and a dot product costs one barrier.  NT threads hold up to E elements
+// each, e = t + NT k; vectors of at most 1024 elements take fewer threads (the
+// 64-element runs of a thread's E elements are separate summands then).
+// Bound: the barriers and the serial scalars.  @MGS@
+template <int L, int NT, int E>
+__global__ __launch_bounds__(NT) void k_mr_mgs_reg(const int32_t *__restrict__ active, Vecs v,
+                                                   Scal sc, int nmu) {
+  // below 1024 threads every element has a column of its own
+  constexpr int NV = NT < kMrThreads ? kMrThreads / NT : 1;
+  static_assert(NT == kMrThreads || E <= NV, "columns of 1024");
+  const int s = blockIdx.x;
+  if (!active[s]) return;
+  __shared__ BlockSum<NT / 64, NV, 4> bs;
+  __shared__ MrLds m;
+  int turn = 0;
+  double2 r[L + 1][E], nu[L + 1];
+#pragma unroll
+  for (int i = 0; i <= L; ++i)
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      const int64_t e = threadIdx.x + (int64_t)k * NT;
+      r[i][k] = e < v.ld ? v.r(s, i)[e] : mk(0, 0);
+    }
+  // sums of a . b and of c . b over the block
+  auto dots = [&](const double2 (&a)[E], const double2 (&c)[E], const double2 (&b)[E],
+                  double2 &ab, double2 &cb) {
+    double p[NV][4], t[4];
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) p[k][q] = 0.0;
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      double(&o)[4] = p[NV > 1 ? k : 0];
+      double2 x = mk(o[0], o[1]), y = mk(o[2], o[3]);
+      cmac(x, a[k], b[k]);
+      cmac(y, c[k], b[k]);
+      o[0] = x.x; o[1] = x.y; o[2] = y.x; o[3] = y.y;
+    }
+    bs.run(p, t, turn);
+    ab = mk(t[0], t[1]);
+    cb = mk(t[2], t[3]);
+  };
+#pragma unroll
+  for (int jj = 1; jj <= L; ++jj) {
+    double2 unused;
+#pragma unroll
+    for (int ii = 1; ii < jj; ++ii) {
+      double2 acc;
+      dots(r[jj], r[jj], r[ii], acc, unused);
+      const double2 t = cdiv(acc, nu[ii]), mt = cneg(t);
+      if (threadIdx.x == 0) m.tau[jj * (jj + 1) / 2 + ii] = t;
+#pragma unroll
+      for (int k = 0; k < E; ++k) cmac(r[jj][k], mt, r[ii][k]);
+    }
+    double2 a2;
+    dots(r[jj], r[0], r[jj], nu[jj], a2);
+    if (threadIdx.x == 0) m.gp[jj] = cdiv(a2, nu[jj]);
+#pragma unroll
+    for (int k = 0; k < E; ++k) {
+      const int64_t e = threadIdx.x + (int64_t)k * NT;
+      if (jj > 1 && e < v.ld) v.r(s, jj)[e] = r[jj][k];
+    }
+  }
+  __syncthreads();
+  mr_scalars<NT>(s, L, v.nsh, nmu, sc, m);
 }
 
 // Convergence test (bicgstab.f90:237,245,296-299) and NaN guard on the
@@ -556,21 +576,38 @@ __global__ __launch_bounds__(NT) void k_mr_mgs(const int32_t *__restrict__ activ
 // (final = 1) a system that has run max_iter of them without converging stops
 // with state 3, iterations max_iter + 1 (the reference's loop variable after
 // DO iter = 1, max_iter, bicgstab.f90:229-253).
-__global__ void k_check(int nsys, const int32_t *__restrict__ count, int max_iter, int final,
-                        double thr, const int32_t *__restrict__ in,
-                        int32_t *__restrict__ out, const double *__restrict__ norm,
-                        int32_t *__restrict__ iters, int32_t *__restrict__ state, Scal sc,
-                        int nsh, int shift_test, double relax_thr, int32_t *__restrict__ relax) {
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= nsys) return;
+// One block per system: the norm of r_0, then the shifted systems over the
+// lanes of its first wavefront.
+__global__ __launch_bounds__(kSumThreads) void k_check(const int32_t *__restrict__ count, int max_iter,
+                                              int final, double thr,
+                                              const int32_t *__restrict__ in,
+                                              int32_t *__restrict__ out, Vecs v,
+                                              int32_t *__restrict__ iters,
+                                              int32_t *__restrict__ state, Scal sc,
+                                              int shift_test, double relax_thr,
+                                              int32_t *__restrict__ relax) {
+  __shared__ BlockSum<kSumThreads / 64, 1, 1> bs;
+  const int s = blockIdx.x, nsh = v.nsh;
   if (!in[s]) {
-    out[s] = 0;
+    if (threadIdx.x == 0) out[s] = 0;
     return;
   }
-  double nr = norm[s];
+  // |r_0|_2
+  const double2 *r0 = v.r(s, 0);
+  double acc[1][1] = {{0.0}}, total[1];
+#pragma unroll 8
+  for (int64_t i = threadIdx.x; i < v.ld; i += kSumThreads) {
+    const double2 x = r0[i];
+    acc[0][0] = fma(x.x, x.x, acc[0][0]);
+    acc[0][0] = fma(x.y, x.y, acc[0][0]);
+  }
+  int turn = 0;
+  bs.run(acc, total, turn);
+  if (threadIdx.x >= 64) return;
+  double nr = sqrt(total[0]);
   if (shift_test) {
     double zmax = 1.0;
-    for (int k = 0; k < nsh; ++k) {
+    for (int k = threadIdx.x; k < nsh; k += 64) {
       if (sc.frozen[s * nsh + k]) continue;
       const double2 z = cmul(sc.inv_theta[s * nsh + k], sc.inv_phi[s * nsh + k]);
       const double az = sqrt(z.x * z.x + z.y * z.y);
@@ -580,8 +617,9 @@ __global__ void k_check(int nsys, const int32_t *__restrict__ count, int max_ite
       if (final && az * nr < 0.5 * thr) sc.frozen[s * nsh + k] = 1;
       else zmax = fmax(zmax, az);
     }
-    nr *= zmax;
+    nr *= lanes::max<64>(zmax);
   }
+  if (threadIdx.x != 0) return;
   // relaxed matrix-vector products (inexact Krylov): once the residual is
   // small the error of an FP32 local-potential FFT, proportional to the
   // vector it multiplies, stays below the final tolerance
@@ -802,15 +840,6 @@ __global__ void k_init_vectors(int nsys, Vecs v, const double2 *__restrict__ rhs
   v.RT[(int64_t)s * v.ld + e] = b;
 }
 
-// x_out[s][k][ldo] <- X (k = 0) or SX (k >= 1)
-__global__ void k_gather_x(Vecs v, double2 *__restrict__ out, int64_t ldo, int64_t n) {
-  const int s = blockIdx.y, k = blockIdx.z;
-  const int64_t e = (int64_t)blockIdx.x * kBlock + threadIdx.x;
-  if (e >= n) return;
-  double2 val = (k == 0) ? v.x(s)[e] : v.sx(s, k - 1)[e];
-  out[((int64_t)s * (v.nsh + 1) + k) * ldo + e] = val;
-}
-
 __global__ void k_nan_scan(int nsys, int nshift, const double2 *__restrict__ x, int64_t ldo,
                            int64_t n, int32_t *__restrict__ has_nan) {
   const int s = blockIdx.x;
@@ -861,7 +890,6 @@ struct BatchBicgstab::Impl {
   DevBuf<double2> R, U, X, RT, SU, SX, RS;
   DevBuf<double2> scal_seed, scal_shift, mu, coef, gam;
   DevBuf<double2> sigma_seed;  // per system seed shift sigma_1
-  DevBuf<double> norms;
   DevBuf<int32_t> active, mr_active, iters, state, count, frozen;
   Scal sc{};
   Vecs vv{};
@@ -987,7 +1015,6 @@ struct BatchBicgstab::Impl {
     mu.alloc(nshs * (l * (l + 1) / 2));
     coef.alloc(nshs * (kMaxL + 2));
     sigma_seed.alloc(S);
-    norms.alloc(S);
     active.alloc(S);
     mr_active.alloc(S);
     iters.alloc(S);
@@ -1085,10 +1112,26 @@ struct BatchBicgstab::Impl {
 
   // ||r_0|| test on the systems of `in`; survivors go to `out`
   void check(hipStream_t st, int max_iter, int final, double thr, int32_t *in, int32_t *out) {
-    k_norm<<<ns, kBlock, 0, st>>>(ns, in, R.p, (l + 1) * ld, ld, norms.p);
-    k_check<<<grid1(ns, 128), 128, 0, st>>>(ns, count.p, max_iter, final, thr, in, out,
-                                               norms.p, iters.p, state.p, sc, nsh, shift_test,
-                                               relax_thr, relax_thr > 0 ? relax.p : nullptr);
+    k_check<<<ns, kSumThreads, 0, st>>>(count.p, max_iter, final, thr, in, out, vv, iters.p,
+                                        state.p, sc, shift_test, relax_thr,
+                                        relax_thr > 0 ? relax.p : nullptr);
+  }
+
+  void mr_part(hipStream_t st, int S) {
+    const int nmu = l * (l + 1) / 2;
+    const int32_t *act = mr_active.p;
+    auto reg = [&](auto ll) {
+      constexpr int L = decltype(ll)::value;
+      if (ld <= 256) k_mr_mgs_reg<L, 256, 1><<<S, 256, 0, st>>>(act, vv, sc, nmu);
+      else if (ld <= 512) k_mr_mgs_reg<L, 256, 2><<<S, 256, 0, st>>>(act, vv, sc, nmu);
+      else if (ld <= 1024) k_mr_mgs_reg<L, 512, 2><<<S, 512, 0, st>>>(act, vv, sc, nmu);
+      else k_mr_mgs_reg<L, 1024, 2><<<S, 1024, 0, st>>>(act, vv, sc, nmu);
+    };
+    if (ld <= 2048 && l == 1) reg(std::integral_constant<int, 1>{});
+    else if (ld <= 2048 && l == 2) reg(std::integral_constant<int, 2>{});
+    else if (ld <= 2048 && l == 3) reg(std::integral_constant<int, 3>{});
+    else if (ld <= 2048 && l == 4) reg(std::integral_constant<int, 4>{});
+    else k_mr_mgs<<<S, kMrThreads, 0, st>>>(act, vv, sc, nmu);
   }
 
   // One outer iteration (bicgstab.f90:229-247) on every active system.  Its
@@ -1098,46 +1141,29 @@ struct BatchBicgstab::Impl {
   void iterate(Operator &op, hipStream_t st, int max_iter, double threshold) {
     const int S = ns;
     const dim3 gv((unsigned)((ld + kBlock - 1) / kBlock), S);
-    const int nmu = l * (l + 1) / 2, ntau = (l + 1) * (l + 2) / 2;
-    const int64_t sstride = (int64_t)(l + 1) * ld;
     // ---- bicg_part (Algorithm 3)
     for (int j = 0; j < l; ++j) {
-      // many slots: each seed half in one launch, one block per system; few
-      // (the lock-step tail): the dot product and the update over a grid of
-      // tiles as two launches, which spreads a system over more CUs.  Both
-      // give the same bits.
-      const bool fused = S >= kFuseHalves;
-      {
+      // each seed half in one launch, one block per system
+      with_threads(ld, [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
         KScope ks_("bicg_v1", st, 2);
-        if (fused) {
-          k_bicg_half1<<<S, kBlock, 0, st>>>(j, active.p, vv, j == 0 ? 1 : 0, 1, sc,
-                                             j == 0 ? fresh.p : nullptr,
-                                             j == 0 ? count.p : nullptr);
-        } else {
-          k_dotu_s1<<<S, kBlock, 0, st>>>(active.p, R.p + j * ld, sstride, RT.p, ld,
-                                          j == 0 ? 1 : 0, 1, sc, j == 0 ? fresh.p : nullptr,
-                                          j == 0 ? count.p : nullptr);
-          k_bicg_v1<<<gv, kBlock, 0, st>>>(j, active.p, vv, sc);
-        }
-      }
+        k_bicg_half1<NT><<<S, NT, 0, st>>>(j, active.p, vv, j == 0 ? 1 : 0, 1, sc,
+                                           j == 0 ? fresh.p : nullptr,
+                                           j == 0 ? count.p : nullptr);
+      });
       op_apply(op, st, U.p + j * ld, U.p + (j + 1) * ld);       // L10
-      {
+      with_threads(ld, [&](auto nt) {
+        constexpr int NT = decltype(nt)::value;
         KScope ks_("bicg_seed", st, 2);
-        if (fused) {
-          k_bicg_half2<<<S, kBlock, 0, st>>>(j, active.p, vv, nsh, l, sc);
-        } else {
-          k_dotu_s2<<<S, kBlock, 0, st>>>(active.p, U.p + (j + 1) * ld, sstride, RT.p, ld, nsh,
-                                          l, j, sc);
-          k_bicg_seed<<<gv, kBlock, 0, st>>>(j, active.p, vv, sc);
-        }
-      }
+        k_bicg_half2<NT><<<S, NT, 0, st>>>(j, active.p, vv, nsh, l, sc);
+      });
       op_apply(op, st, R.p + j * ld, R.p + (j + 1) * ld);       // L24
     }
     check(st, max_iter, 0, threshold, active.p, mr_active.p);
     // ---- mr_part (Algorithm 4) on the systems still running
     {
       KScope ks_("mr_mgs", st, 2);
-      k_mr_mgs<1024><<<S, 1024, 0, st>>>(mr_active.p, vv, sc, ntau, nmu);
+      mr_part(st, S);
     }
     if (nsh > 0) {  // the shifted systems: BiCG half of this iteration and, if running, MR half
       KScope ks_("shift_cycle", st, 2);
