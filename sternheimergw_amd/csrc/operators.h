@@ -135,6 +135,9 @@ class PwOperator : public Operator {
   // last column holding plane waves; ncs_ columns per plane) and the full
   // grid (nslot_ columns, the layout of every other kernel)
   int ncs_ = 0;
+  // columns per plane that T and S need: the grid of the sphere's own
+  // half-widths, at least ncs_ (nslot_ may count one half-width for all axes)
+  int64_t box_cols_ = 0;
   DevBuf<int4> pk_info_, gr_info_;
   DevBuf<int32_t> pk_row_start_, pk_row_lo_, pk_row_cnt_;
   DevBuf<int32_t> gr_row_start_, gr_row_lo_, gr_row_cnt_;

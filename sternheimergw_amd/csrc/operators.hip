@@ -930,14 +930,14 @@ __global__ __launch_bounds__(64) void k_pw_plane_grad(PwDev d, const double2 *__
 constexpr int kChunk = 64;
 constexpr int kVT = 16;
 constexpr int kAsmChunk = 64, kAsmThreads = 256;  // k_pw_assemble2 default block shape
-constexpr int kPT = 16;  // projectors staged in LDS at a time
 
 // does any vector of the tile still run?  (uniform across the block)
 __device__ inline bool tile_active(const int32_t *__restrict__ active,
                                    const int32_t *__restrict__ vecs, int nv) {
-  int any = 0;
-  for (int k = 0; k < nv; ++k) any |= active[vecs[k]];
-  return any != 0;
+  // one vector to a lane: taken in turn, each costs two dependent loads (a
+  // small batch's assembly 14.7 us against 13.6)
+  const int lane = threadIdx.x & 63;
+  return __any(lane < nv && active[vecs[lane]] != 0);
 }
 
 // becp[g][vt][p][vl] = D_p sum over the chunk partials (once per tile); one
@@ -1019,31 +1019,96 @@ __device__ inline void becp_body(const PwDev &d, const double2 *__restrict__ in,
   if (v0 >= cnt || i0 >= npw) return;
   const int nv = min(kVT, cnt - v0), lim = min(kChunk, npw - i0), nproj = d.nproj;
   if (active && !tile_active(active, gvec + g * maxper + v0, nv)) return;
+  // A sum runs over the chunk's plane waves in order, whatever the tiling.  Up
+  // to 16 projectors: one sum to a lane, the whole chunk staged at once (a few
+  // vectors of the 32^3 box, 16 projectors: 33.9 us an application against 35.3
+  // in four stages).  More: wave w takes 16 of 64 projectors, a lane 2 x 2 of
+  // their 16 x 16 (projector, vector) sums, one operand read from LDS a product
+  // where one sum per lane takes two; the plane waves come 16 at a time.  On
+  // the 48^3 box (72 projectors, 512 vectors) with the z transforms beside it
+  // 16.8 us a launch against 21.6 with one sum to a lane.
+  // Loads are unconditional, their places clamped: under a condition each is
+  // waited for by itself.
+  constexpr int kIB = 16, kPB = 64;
+  static_assert(kVT == 16 && kChunk % kIB == 0, "256 lanes: 4 waves of 8 x 8 lanes");
   __shared__ double2 xs[kVT][kChunk + 1];
-  __shared__ double2 ps[kPT][kChunk + 1];
-  for (int t = threadIdx.x; t < kVT * kChunk; t += 256) {
-    const int vl = t / kChunk, i = t % kChunk;
-    double2 val = mk(0, 0);
-    if (vl < nv && i < lim) {
-      const int v = gvec[g * maxper + v0 + vl];
-      if (!active || active[v]) val = in[v * sin + i0 + i];
-    }
-    xs[vl][i] = val;
-  }
+  __shared__ double2 ps[kPB][kIB + 1];
+  static_assert(kPB * (kIB + 1) >= 16 * (kChunk + 1), "16 whole rows");
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   const double2 *pg = d.proj + (int64_t)g * nproj * d.ld + i0;
   double2 *pout = part + (((int64_t)g * tiles + vt) * nchunk + chunk) * nproj * kVT;
-  for (int p0 = 0; p0 < nproj; p0 += kPT) {
+  const int npb = (nproj + kPB - 1) / kPB;
+  const bool few = nproj <= 16;
+  double2 next[4];
+  auto load = [&](int p, int i) {
+    const double2 q = pg[(int64_t)min(p, nproj - 1) * d.ld + min(i, lim - 1)];
+    const bool in = p < nproj && i < lim;
+    return mk(in ? q.x : 0.0, in ? q.y : 0.0);
+  };
+  auto fetch = [&](int stage) {  // stage = projector block, then plane-wave block
+    const int p0 = stage / (kChunk / kIB) * kPB, ib = stage % (kChunk / kIB) * kIB;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) next[r] = load(p0 + tid / kIB + 16 * r, ib + tid % kIB);
+  };
+  if (few) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) next[r] = load(wv + 4 * r, lane);
+  } else {
+    fetch(0);
+  }
+#pragma unroll
+  for (int r = 0; r < kVT / 4; ++r) {
+    const int vl = wv + 4 * r;  // uniform over the wave
+    const int v = gvec[g * maxper + v0 + min(vl, nv - 1)];
+    const double2 val = in[v * sin + i0 + min(lane, lim - 1)];
+    const bool on = vl < nv && lane < lim && (!active || active[v]);
+    xs[vl][lane] = mk(on ? val.x : 0.0, on ? val.y : 0.0);
+  }
+  if (few) {
+    double2 *rows = &ps[0][0];  // [16][kChunk + 1]
+#pragma unroll
+    for (int r = 0; r < 4; ++r) rows[(wv + 4 * r) * (kChunk + 1) + lane] = next[r];
     __syncthreads();
-    for (int t = threadIdx.x; t < kPT * kChunk; t += 256) {
-      const int pl = t / kChunk, i = t % kChunk;
-      ps[pl][i] = (p0 + pl < nproj && i < lim) ? pg[(int64_t)(p0 + pl) * d.ld + i] : mk(0, 0);
-    }
-    __syncthreads();
-    const int o = threadIdx.x;  // kPT * kVT == 256 outputs
-    const int pl = o / kVT, vl = o % kVT;
+    const int p = tid / kVT, vl = tid % kVT;
     double2 acc = mk(0, 0);
-    for (int i = 0; i < lim; ++i) cmacc(acc, ps[pl][i], xs[vl][i]);
-    if (p0 + pl < nproj) pout[(p0 + pl) * kVT + vl] = acc;
+    for (int i = 0; i < lim; ++i) cmacc(acc, rows[p * (kChunk + 1) + i], xs[vl][i]);
+    if (p < nproj) pout[p * kVT + vl] = acc;
+    return;
+  }
+  const int tp = 16 * wv + (lane >> 3), tv = lane & 7;
+  for (int pb = 0; pb < npb; ++pb) {
+    const bool mine = pb * kPB + 16 * wv < nproj;  // uniform over the wave
+    double2 acc[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) acc[a][b] = mk(0, 0);
+    for (int ib = 0; ib < kChunk; ib += kIB) {
+      const int stage = pb * (kChunk / kIB) + ib / kIB;
+      if (stage > 0) __syncthreads();
+#pragma unroll
+      for (int r = 0; r < 4; ++r) ps[tid / kIB + 16 * r][tid % kIB] = next[r];
+      __syncthreads();
+      if (stage + 1 < npb * (kChunk / kIB)) fetch(stage + 1);
+      if (mine) {
+#pragma unroll
+        for (int i = 0; i < kIB; ++i) {
+          const double2 pa = ps[tp][i], pb2 = ps[tp + 8][i];
+          const double2 xa = xs[tv][ib + i], xb = xs[tv + 8][ib + i];
+          cmacc(acc[0][0], pa, xa);
+          cmacc(acc[0][1], pa, xb);
+          cmacc(acc[1][0], pb2, xa);
+          cmacc(acc[1][1], pb2, xb);
+        }
+      }
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        const int p = pb * kPB + tp + 8 * a;
+        if (p < nproj) pout[p * kVT + tv + 8 * b] = acc[a][b];
+      }
   }
 }
 
@@ -1065,13 +1130,6 @@ __global__ __launch_bounds__(NT) void k_pw_assemble2(
   if (v0 >= cnt) return;
   const int nv = min(kVT, cnt - v0), nproj = d.nproj, n3 = d.n3;
   const int npw = d.npw[g], i0 = chunk * CH;
-  if (active && !tile_active(active, gvec + g * maxper + v0, nv)) return;
-  double2 *becp = smem;            // [nproj][kVT]
-  double2 *w3 = becp + nproj * kVT;  // n3
-  const double2 *bsrc = part + ((int64_t)g * tiles + vt) * nproj * kVT;  // reduced D becp
-  for (int o = threadIdx.x; o < nproj * kVT; o += NT) becp[o] = bsrc[o];
-  for (int i = threadIdx.x; i < n3; i += NT) w3[i] = d.tw3[i];
-  __syncthreads();
   // thread = (plane wave i of the chunk, vector quarter vq): vectors
   // vl = vq + 4k, k < 4, accumulate together so each projector value is
   // loaded once per thread
@@ -1080,35 +1138,43 @@ __global__ __launch_bounds__(NT) void k_pw_assemble2(
   static_assert(kVT % kVQ == 0, "vector groups must divide the tile");
   const int i = threadIdx.x % CH, vq = threadIdx.x / CH;
   const int64_t e = (int64_t)i0 + i;
-  if (e >= d.ld) return;
-  const double2 *pg = d.proj + (int64_t)g * nproj * d.ld;
-  const int64_t ge = (int64_t)g * d.ld + e;
+  const bool inside = e < npw;
+  // kAhead projector values are loaded together, the first from before the
+  // overlaps are in LDS.  The loads are unconditional (past the last projector
+  // they repeat it): under a condition each would be waited for by itself.
+  // A second set in flight (16 + 16) costs a wavefront per SIMD: 18.4 us per
+  // launch of the streamed 48^3 solve against 15.0.
+  constexpr int kAhead = 8;
+  const double2 *pg = d.proj + (int64_t)g * nproj * d.ld + (inside ? e : 0);
+  double2 pv[kAhead];
+  auto fetch = [&](int p0) {
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q) pv[q] = pg[(int64_t)min(p0 + q, nproj - 1) * d.ld];
+  };
+  if (nproj > 0) fetch(0);
+  if (active && !tile_active(active, gvec + g * maxper + v0, nv)) return;
+  double2 *becp = smem;            // [nproj][kVT]
+  const double2 *bsrc = part + ((int64_t)g * tiles + vt) * nproj * kVT;  // reduced D becp
+  for (int o = threadIdx.x; o < nproj * kVT; o += NT) becp[o] = bsrc[o];
+  const int64_t ge = (int64_t)g * d.ld + (inside ? e : 0);
+  const double kin = d.kin[ge];
   int vv[kPer];
   bool on[kPer];
+  bool any = false;
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
     const int vl = vq + kVQ * k;
     on[k] = vl < nv;
     vv[k] = on[k] ? gvec[g * maxper + v0 + vl] : 0;
     if (on[k] && active && !active[vv[k]]) on[k] = false;
+    any |= on[k];
   }
-  bool any = false;
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) any |= on[k];
-  if (!any) return;  // no running vector in this thread's group
-  if (e >= npw) {  // padding stays zero
-#pragma unroll
-    for (int k = 0; k < kPer; ++k)
-      if (on[k]) out[vv[k] * sout + e] = mk(0, 0);
-    return;
-  }
-  const double kin = d.kin[ge];
   double2 xi[kPer], acc[kPer];
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
-    xi[k] = on[k] ? in[vv[k] * sin + e] : mk(0, 0);
+    xi[k] = on[k] && inside ? in[vv[k] * sin + e] : mk(0, 0);
     acc[k] = mk(kin * xi[k].x, kin * xi[k].y);
-    if (!on[k]) continue;
+    if (!on[k] || !inside) continue;
     if (locv) {  // z transform done by k_pw_zfwd (already scaled)
       const double2 l = locv[vv[k] * d.ld + e];
       acc[k].x += l.x;
@@ -1117,15 +1183,27 @@ __global__ __launch_bounds__(NT) void k_pw_assemble2(
       const double2 *col = S + ((int64_t)vv[k] * d.nslot + d.slot_of[ge]) * n3;
       const int mz = d.m3_of[ge];
       double2 loc = mk(0, 0);
-      for (int z = 0; z < n3; ++z) cmac(loc, col[z], cconj(w3[(mz * z) % n3]));
+      for (int z = 0; z < n3; ++z) cmac(loc, col[z], cconj(d.tw3[(mz * z) % n3]));
       acc[k].x = fma(loc.x, d.inv_nbox, acc[k].x);
       acc[k].y = fma(loc.y, d.inv_nbox, acc[k].y);
     }
   }
-  for (int p = 0; p < nproj; ++p) {
-    const double2 pv = pg[(int64_t)p * d.ld + e];
+  __syncthreads();
+  if (!any || e >= d.ld) return;  // no running vector in this thread's group
+  if (!inside) {  // padding stays zero
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) cmac(acc[k], pv, becp[p * kVT + vq + kVQ * k]);
+    for (int k = 0; k < kPer; ++k)
+      if (on[k]) out[vv[k] * sout + e] = mk(0, 0);
+    return;
+  }
+  for (int p0 = 0; p0 < nproj; p0 += kAhead) {
+#pragma unroll
+    for (int q = 0; q < kAhead; ++q)
+      if (p0 + q < nproj) {
+#pragma unroll
+        for (int k = 0; k < kPer; ++k) cmac(acc[k], pv[q], becp[(p0 + q) * kVT + vq + kVQ * k]);
+      }
+    if (p0 + kAhead < nproj) fetch(p0 + kAhead);
   }
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
@@ -1145,14 +1223,16 @@ template <int... Ms, typename F> inline bool dispatch_band(int m, F &&f) {
 // f(std::integral_constant<int, M>) with M = m when m is one of the sphere
 // half-widths specialised for box N (the usual ones: the box is the smallest
 // FFT size of at least 4M + 1, or one size up), else with M = -1
+constexpr int kBandMin = 4;
+constexpr int band_max(int n) {
+  return n == 48 ? 11 : n == 36 ? 8 : n == 32 ? 7 : n == 24 ? 5 : -1;
+}
 template <int N, typename F> inline void with_band(bool enable, int m, F &&f) {
   bool hit = false;
-  if (enable) {
-    if constexpr (N == 48) hit = dispatch_band<8, 9, 10, 11>(m, f);
-    if constexpr (N == 36) hit = dispatch_band<7, 8>(m, f);
-    if constexpr (N == 32) hit = dispatch_band<6, 7>(m, f);
-    if constexpr (N == 24) hit = dispatch_band<4, 5>(m, f);
-  }
+  if (enable)
+    [&]<int... I>(std::integer_sequence<int, I...>) {
+      hit = dispatch_band<kBandMin + I...>(m, f);
+    }(std::make_integer_sequence<int, std::max(0, band_max(N) - kBandMin + 1)>{});
   if (!hit) f(std::integral_constant<int, -1>{});
 }
 
@@ -1340,6 +1420,27 @@ static std::vector<double2> twiddles(int n) {
 
 static inline int modn(int a, int n) { return ((a % n) + n) % n; }
 
+// does every column (m1, m2) of every group hold a run of m3 without gaps?
+static bool whole_columns(const PwDesc &desc, int M1, int M2) {
+  const int nc2 = 2 * M2 + 1;
+  std::vector<int32_t> lo, hi, cnt;
+  for (int g = 0; g < desc.ngroup; ++g) {
+    lo.assign((size_t)(2 * M1 + 1) * nc2, INT32_MAX);
+    hi.assign(lo.size(), INT32_MIN);
+    cnt.assign(lo.size(), 0);
+    for (int i = 0; i < desc.npw[g]; ++i) {
+      const int32_t *m = desc.mill + ((int64_t)g * desc.ld + i) * 3;
+      const size_t c = (size_t)(m[0] + M1) * nc2 + (m[1] + M2);
+      lo[c] = std::min(lo[c], m[2]);
+      hi[c] = std::max(hi[c], m[2]);
+      ++cnt[c];
+    }
+    for (size_t c = 0; c < cnt.size(); ++c)
+      if (cnt[c] > 0 && hi[c] - lo[c] + 1 != cnt[c]) return false;
+  }
+  return true;
+}
+
 PwOperator::PwOperator(const PwDesc &desc) {
   n1_ = desc.n1; n2_ = desc.n2; n3_ = desc.n3;
   if (const char *f = std::getenv("SGW_PW_FUSE")) fuse_stages_ = std::strcmp(f, "0") != 0;
@@ -1367,6 +1468,17 @@ PwOperator::PwOperator(const PwDesc &desc) {
   SGW_REQUIRE(2 * M1 + 1 <= n1_ && 2 * M2 + 1 <= n2_ && 2 * M3 + 1 <= n3_, SGW_E_SHAPE,
               "pw operator: the plane-wave sphere does not fit in the FFT box");
   n = npw_[0];
+  box_cols_ = (int64_t)(2 * M1 + 1) * (2 * M2 + 1);
+  const int M = std::max(M1, std::max(M2, M3));
+  if (n1_ == n2_ && n2_ == n3_ && band_planes_ && split_planes_ && fuse_stages_ &&
+      M >= kBandMin && M <= band_max(n1_) && whole_columns(desc, M1, M2)) {
+    // the transforms specialised to a half-width take one for all axes, and a
+    // k+q shift often leaves the three one apart; the rows this adds hold no
+    // columns, and the packed layout that these transforms use has no places
+    // for them.  512 vectors of the 48^3 box at half-widths (9, 8, 9): 254 us
+    // against 319 without, at (7, 6, 7) 210 against 292
+    M1 = M2 = M3 = M;
+  }
   M1_ = M1; M2_ = M2; M3_ = M3;
   nc1_ = 2 * M1 + 1; nc2_ = 2 * M2 + 1;
   nslot_ = nc1_ * nc2_;
@@ -1779,7 +1891,7 @@ void PwOperator::apply_work(hipStream_t st, int nvec, const double2 *in, int64_t
   }
   SGW_HIP(hipGetLastError());
   {
-    const size_t lds_asm = sizeof(double2) * ((size_t)nproj_ * kVT + n3_);
+    const size_t lds_asm = sizeof(double2) * (size_t)nproj_ * kVT;
     KScope ks("pw_assemble", st, 2);
     // 64 plane waves x 4 vector groups per 256-lane block by default: on the
     // 48^3 batch 21.9 us per 512 vectors against 26.4 with 32 plane waves x 8
@@ -2015,7 +2127,7 @@ void PwOperator::apply_noalloc(hipStream_t st, int nvec, const int32_t *d_group,
   const size_t b_plan = align256(sizeof(int32_t) * ((size_t)ngroup_ * maxper + ngroup_));
   const size_t b_part = align256(sizeof(double2) * (size_t)ngroup_ * tiles * nchunk * np * kVT);
   const size_t b_becp = align256(sizeof(double2) * (size_t)ngroup_ * tiles * np * kVT);
-  const size_t b_box = align256(sizeof(double2) * (size_t)nvec * nslot_ * n3_);
+  const size_t b_box = align256(sizeof(double2) * (size_t)nvec * box_cols_ * n3_);
   const size_t b_loc = align256(sizeof(double2) * (size_t)nvec * ld);
   const size_t b_vlist = align256(sizeof(int32_t) * (size_t)nvec);
   const size_t total = b_plan + b_part + b_becp + 2 * b_box + b_loc + b_vlist;
