@@ -50,6 +50,16 @@ template <int O> __device__ inline Pair step(double v) {
           __longlong_as_double(((long long)hi.b << 32) | (unsigned int)lo.b)};
 }
 
+// a of the upper 32 lanes and b of the lower 32 change places
+__device__ inline void swap_halves(double &a, double &b) {
+  const long long x = __double_as_longlong(a), y = __double_as_longlong(b);
+  const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)x, (unsigned)y, false, false);
+  const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)(x >> 32), (unsigned)(y >> 32), false,
+                                                   false);
+  a = __longlong_as_double(((long long)hi[0] << 32) | (unsigned int)lo[0]);
+  b = __longlong_as_double(((long long)hi[1] << 32) | (unsigned int)lo[1]);
+}
+
 template <int O, typename T, typename F> __device__ inline T fold(T v, F f) {
   if constexpr (O == 0) {
     return v;

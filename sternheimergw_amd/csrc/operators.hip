@@ -12,6 +12,8 @@
 //                     with D = alpha_pv, the valence states of P_v.
 #include "operators.h"
 #include "ktimer.h"
+#include "lanes.h"
+#include "lines.h"
 #include "regfft.h"
 #include "splitfft.h"
 #include "tune.h"
@@ -885,39 +887,86 @@ __global__ __launch_bounds__(128, 2) void k_pw_plane_drho_split(PwDev d,
 
 // Adjoint gradient of one z-plane over a strided set of vector pairs:
 //   G[b][z][x][y] += sum_{p = b, b + nb, ...} w_p Re(conj(y_p(r)) x_p(r)),
-// from the z-transformed columns Tx (x_p) and Ty (y_p).  Block (z, b) owns
-// its plane of G exclusively; the x plane waits in LDS (Xs[x][y]) for y.
-template <int N>
-__global__ __launch_bounds__(64) void k_pw_plane_grad(PwDev d, const double2 *__restrict__ Tx,
-                                                      const double2 *__restrict__ Ty, int np,
-                                                      const double *__restrict__ w,
-                                                      double *__restrict__ G, int accumulate) {
+// from the z-transformed columns Tx (x_p) and Ty (y_p) in the packed layout
+// (d.col_info).  Block (z, b) owns its plane of G, which stays in registers
+// over its pairs.  The lower 32 lanes of a wave transform x and the upper 32
+// y, every line over a lane pair: 16 rows or columns of both to a wave, so
+// one pass of ceil(N/16) waves takes all of them; a swap of the wave's halves
+// then leaves the same points of x and y in one lane.
+//   Bound: the latency of the two transforms and their LDS exchange, between
+// two barriers a pair, at three quarters of the adds' own time.  2 048 pairs of
+// the 48^3 box (half-width 4): 638 us against 2 673 with whole lines in one
+// lane, x waiting in LDS and G read and written for every pair.
+// MB as in plane_split_body.
+constexpr int grad_waves(int n) { return (n + 15) / 16; }
+template <int N, int MB>
+__global__ __launch_bounds__(64 * grad_waves(N), 3) void k_pw_plane_grad(
+    PwDev d, const double2 *__restrict__ Tx, const double2 *__restrict__ Ty, int np,
+    const int32_t *__restrict__ group, const double *__restrict__ w, double *__restrict__ G,
+    int accumulate) {
+  constexpr int E = N / 2, F = N / 4, R = N + 1;
   extern __shared__ double2 smem[];
-  const int z = blockIdx.x, b = blockIdx.y, nb = gridDim.y;
-  const int lane = threadIdx.x;
-  double2 *T = smem;               // nslot
-  double2 *P = T + d.nslot;        // nc1 * N
-  double2 *Xs = P + d.nc1 * N;     // N * N
-  double *Gz = G + ((int64_t)b * N + z) * N * N;
-  if (!accumulate && lane < N)
-    for (int x = 0; x < N; ++x) Gz[(int64_t)x * N + lane] = 0.0;
-  double2 buf[N];
-  for (int p = b; p < np; p += nb) {
-    plane_to_real<N>(d, Tx + ((int64_t)p * N + z) * d.nslot, T, P, buf);
-    if (lane < N)
+  const int z = blockIdx.x, b0 = blockIdx.y, nb = gridDim.y;
+  const int lane = threadIdx.x & 63, half = lane >> 5;
+  const int r = (threadIdx.x >> 6) * 16 + ((lane & 31) >> 1);
+  const Line<N> ln{lane & 1};
+  const int nc1 = MB >= 0 ? 2 * MB + 1 : d.nc1, M1 = MB >= 0 ? MB : d.M1;
+  const int ncs = d.ncs;
+  double2 *P = smem + half * nc1 * R;  // rows of x, then rows of y
+  const double2 *T = half ? Ty : Tx;
+  auto freq = [](int i) { return i < N / 2 ? i : i - N; };
+  // G[x][y] at y = r, x = nat(i + F half)
+  double *Gz = G + ((int64_t)b0 * N + z) * N * N + r;
+  double acc[F];
 #pragma unroll
-      for (int x = 0; x < N; ++x) Xs[x * N + lane] = buf[x];
-    plane_to_real<N>(d, Ty + ((int64_t)p * N + z) * d.nslot, T, P, buf);
-    if (lane < N) {
+  for (int i = 0; i < F; ++i) acc[i] = 0.0;
+  auto at = [&](int i) { return (int64_t)(half ? ln.nat(i + F) : ln.nat(i)) * N; };
+  if (accumulate && r < N)
+#pragma unroll
+    for (int i = 0; i < F; ++i) acc[i] = Gz[at(i)];
+  for (int p = b0; p < np; p += nb) {
+    if (r < nc1) {  // Y inverse of row r
+      const int g = group ? group[p] : 0;
+      const int64_t gr = (int64_t)g * nc1 + r;
+      const int lo = d.row_lo[gr], cnt = d.row_cnt[gr];
+      // an empty row reads the plane's first column and keeps nothing of it
+      const double2 *row = T + ((int64_t)p * N + z) * ncs + (cnt > 0 ? d.row_start[gr + g] : 0);
+      double2 b[E];
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        // off the band both points of a pair of lanes are, at compile time
+        const bool band = MB < 0 || 2 * i <= MB || 2 * i + 1 >= N - MB;
+        const int k = freq(ln.dec(i)) - lo;
+        b[i] = band ? keep(row[within(k, cnt)], k, cnt) : mk(0, 0);
+      }
+      ln.template dit<+1>(b);
+      double2 *Pr = P + r * R;
+#pragma unroll
+      for (int i = 0; i < E; ++i) Pr[ln.nat(i)] = b[i];
+    }
+    __syncthreads();
+    if (r < N) {  // X inverse of column y = r
+      double2 b[E];
+#pragma unroll
+      for (int i = 0; i < E; ++i) {
+        const bool band = MB < 0 || 2 * i <= MB || 2 * i + 1 >= N - MB;
+        const int a = freq(ln.dec(i)) + M1;
+        b[i] = band ? keep(P[within(a, nc1) * R + r], a, nc1) : mk(0, 0);
+      }
+      ln.template dit<+1>(b);
       const double wp = w[p];
 #pragma unroll
-      for (int x = 0; x < N; ++x) {
-        const double2 a = Xs[x * N + lane];
-        double *g = Gz + (int64_t)x * N + lane;
-        *g = fma(wp, buf[x].x * a.x + buf[x].y * a.y, *g);
+      for (int i = 0; i < F; ++i) {
+        lanes::swap_halves(b[i].x, b[i + F].x);
+        lanes::swap_halves(b[i].y, b[i + F].y);
+        acc[i] = fma(wp, b[i + F].x * b[i].x + b[i + F].y * b[i].y, acc[i]);
       }
     }
+    __syncthreads();
   }
+  if (r < N)
+#pragma unroll
+    for (int i = 0; i < F; ++i) Gz[at(i)] = acc[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -930,6 +979,18 @@ __global__ __launch_bounds__(64) void k_pw_plane_grad(PwDev d, const double2 *__
 constexpr int kChunk = 64;
 constexpr int kVT = 16;
 constexpr int kAsmChunk = 64, kAsmThreads = 256;  // k_pw_assemble2 default block shape
+
+// columns of nvec vectors of x and of as many of y (blockIdx.z) along z
+template <int N, int MB>
+__global__ __launch_bounds__(64) void k_pw_zinv_pair(PwDev d, const double2 *__restrict__ x,
+                                                     const double2 *__restrict__ y, int64_t sin,
+                                                     const int32_t *__restrict__ group,
+                                                     double2 *__restrict__ Tx,
+                                                     double2 *__restrict__ Ty) {
+  zinv_split_body<N, MB>(d, blockIdx.z ? y : x, sin, group, nullptr, blockIdx.z ? Ty : Tx,
+                         blockIdx.y, blockIdx.x * 32 + (int)(threadIdx.x >> 1),
+                         (threadIdx.x & 1) != 0);
+}
 
 // does any vector of the tile still run?  (uniform across the block)
 __device__ inline bool tile_active(const int32_t *__restrict__ active,
@@ -1983,8 +2044,10 @@ void PwOperator::grad_accumulate(hipStream_t st, int np, const double2 *x, const
   const bool cubic = n1_ == n2_ && n2_ == n3_ && columns_contiguous_;
   SGW_REQUIRE(cubic && (n1_ == 24 || n1_ == 32 || n1_ == 36 || n1_ == 48), SGW_E_ARG,
               "pw operator: the V_loc gradient needs a cubic 24/32/36/48 box");
-  const size_t lds = sizeof(double2) * (nslot_ + (size_t)nc1_ * n1_ + (size_t)n1_ * n1_);
-  SGW_REQUIRE(lds <= 64 * 1024, SGW_E_ARG, "pw operator: gradient plane does not fit in LDS");
+  SGW_REQUIRE(sizeof(double2) * (nslot_ + (size_t)nc1_ * n1_ + (size_t)n1_ * n1_) <= 64 * 1024,
+              SGW_E_ARG, "pw operator: gradient plane does not fit in LDS");
+  // at most 40 KB by the line above
+  const size_t lds = sizeof(double2) * 2 * (size_t)nc1_ * (n1_ + 1);
   SGW_REQUIRE(nb >= 1 && nb < 65536, SGW_E_ARG, "pw operator: bad gradient partial count");
   ensure_scratch(np);
   PwDev d;
@@ -1995,18 +2058,20 @@ void PwOperator::grad_accumulate(hipStream_t st, int np, const double2 *x, const
   d.col_start = col_start_.p; d.col_cnt = col_cnt_.p;
   d.sorted_idx = sidx_.p; d.sorted_m3 = sm3_.p; d.slot_of = slot_of_.p; d.m3_of = m3_of_.p;
   d.col_lo = col_lo_.p;
-  d.ncs = nslot_; d.col_info = gr_info_.p;
-  d.row_start = gr_row_start_.p; d.row_lo = gr_row_lo_.p; d.row_cnt = gr_row_cnt_.p;
+  d.ncs = ncs_; d.col_info = pk_info_.p;
+  d.row_start = pk_row_start_.p; d.row_lo = pk_row_lo_.p; d.row_cnt = pk_row_cnt_.p;
   d.kin = kin_.p; d.proj = proj_.p; d.dcoef = dcoef_.p;
   d.tw1 = tw_.p; d.tw2 = tw_.p + n1_; d.tw3 = tw_.p + n1_ + n2_;
   d.inv_nbox = 1.0 / ((double)n1_ * n2_ * n3_);
-  const dim3 gcol((unsigned)((nslot_ + 63) / 64), np);
+  const dim3 gcol((unsigned)((ncs_ + 31) / 32), np, 2);
   auto run = [&](auto tag) {
     constexpr int NB = decltype(tag)::value;
-    k_pw_zinv<NB><<<gcol, 64, 0, st>>>(d, x, stride, d_group, nullptr, T_.p);
-    k_pw_zinv<NB><<<gcol, 64, 0, st>>>(d, y, stride, d_group, nullptr, S_.p);
-    k_pw_plane_grad<NB><<<dim3(NB, nb), 64, lds, st>>>(d, T_.p, S_.p, np, d_w, G,
-                                                       accumulate ? 1 : 0);
+    with_band<NB>(band_planes_ && M1_ == M2_ && M1_ == M3_, M1_, [&](auto mb) {
+      constexpr int MB = decltype(mb)::value;
+      k_pw_zinv_pair<NB, MB><<<gcol, 64, 0, st>>>(d, x, y, stride, d_group, T_.p, S_.p);
+      k_pw_plane_grad<NB, MB><<<dim3(NB, nb), 64 * grad_waves(NB), lds, st>>>(
+          d, T_.p, S_.p, np, d_group, d_w, G, accumulate ? 1 : 0);
+    });
   };
   switch (n1_) {
     case 24: run(std::integral_constant<int, 24>{}); break;

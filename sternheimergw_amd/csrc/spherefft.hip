@@ -18,8 +18,7 @@
 #include <cstring>
 
 #include "ktimer.h"
-#include "regfft.h"
-#include "splitfft.h"
+#include "lines.h"
 
 namespace sgw {
 namespace {
@@ -28,13 +27,8 @@ enum { kInv = 0, kFwd = 1, kProd = 2 };
 constexpr int kLdsMax = 160 * 1024;
 constexpr int kPre = 2;  // list values a thread fetches ahead for its next box
 
-// Sides divisible by four split every line over a lane pair (splitfft.h): half
-// the registers per lane, so twice the waves hide the LDS exchanges between
-// the stages.  Other sides keep a line in one lane.
-constexpr bool split_side(int n) { return n % 4 == 0; }
 constexpr int planes_per_wave(int n) { return (split_side(n) ? 32 : 64) / n; }
-// values of a line in one lane, and the dwords their index bytes take
-constexpr int lane_values(int n) { return split_side(n) ? n / 2 : n; }
+// dwords the index bytes of a lane's values take
 constexpr int map_dwords(int n) { return (lane_values(n) + 3) / 4; }
 // bytes of an index table of one line: both lanes of a pair, or one lane
 constexpr int map_bytes(int n) { return 4 * map_dwords(n) * (split_side(n) ? 2 : 1); }
@@ -75,25 +69,6 @@ int blocks_per_cu(int n, size_t lds) {
   return std::max(1, std::min((int)(kLdsMax / ((lds + grain - 1) / grain * grain)),
                               4 * waves_per_simd(n) / waves_of(n)));
 }
-
-// A line's values in this lane: value i is point dec(i) of a transform's
-// decimated side and point nat(i) of its natural side; dit goes from the
-// first to the second, dif back.
-template <int N> struct Line {
-  static constexpr bool S = split_side(N);
-  static constexpr int E = lane_values(N), H = N / 2, Q = N / 4;
-  int odd;
-  __device__ int dec(int i) const { return S ? 2 * i + odd : i; }
-  __device__ int nat(int i) const { return S ? (i < Q ? i : H + i - Q) + Q * odd : i; }
-  template <int SIGN> __device__ void dit(double2 (&x)[E]) const {
-    if constexpr (S) split_dit<N, SIGN>(x, odd);
-    else reg_fft<N, SIGN>(x);
-  }
-  template <int SIGN> __device__ void dif(double2 (&x)[E]) const {
-    if constexpr (S) split_dif<N, SIGN>(x, odd);
-    else reg_fft<N, SIGN>(x);
-  }
-};
 
 __device__ inline unsigned map_byte(const uint32_t *m, int i) {
   return (m[i / 4] >> (8 * (i & 3))) & 0xffu;

@@ -10,7 +10,10 @@ of 3 x 48 points and sums of up to 2 000 products stays below 1e-13, 1e-12 is
 asked for.  A vector's result does not depend on the batch it is in, bit for
 bit.
 
-Solver: vector lengths around the thread counts of its kernels, l = 1 .. 5."""
+Solver: vector lengths around the thread counts of its kernels, l = 1 .. 5.
+
+Gradient: every box, several k+q groups, more and fewer pairs than partial
+planes."""
 import ctypes
 import dataclasses
 import types
@@ -19,8 +22,9 @@ import numpy as np
 import pytest
 import torch
 
+from oracle import adjoint_oracle as ao
 from oracle import oracle as orc
-from sternheimergw_amd import _lib, cell, operators
+from sternheimergw_amd import _lib, batch, cell, operators
 
 pytestmark = pytest.mark.gpu
 
@@ -141,3 +145,26 @@ def test_solver_lengths(n):
             for k in range(sig.size):
                 r = a @ x[s, k] + sig[k] * x[s, k] - b[s]
                 assert np.linalg.norm(r) <= 1e-10 * np.linalg.norm(b[s]), (l, s, k)
+
+
+@pytest.mark.parametrize("n,nq,nshift", [(24, 2, 3), (32, 2, 3), (36, 3, 2), (48, 2, 2),
+                                          (24, 1, 40)])
+def test_gradient_boxes(n, nq, nshift):
+    w = cell.workload_c5(nq=nq, nbnd=1, nshift=nshift, ng=2, box=(n, n, n))
+    print(f"gradient {n}^3: {w.nsys} systems x {w.nshift} shifts", flush=True)
+    rng = np.random.Generator(np.random.PCG64(n))
+    weight = rng.uniform(0.2, 1.0, (w.nsys, w.nshift))
+    op = operators.PwOperator.from_workload(w)
+    sol = batch.BatchSolver(op, w.nsys, w.nshift, w.ld, lmax=4, threshold=1e-12, shift_test=True)
+    d = {k: torch.from_numpy(np.ascontiguousarray(v)).to(DEV)
+         for k, v in dict(g=w.group, b=w.rhs, s=w.sigma, w=weight).items()}
+    x = torch.zeros((w.nsys, w.nshift, w.ld), dtype=torch.complex128, device=DEV)
+    y = torch.zeros_like(x)
+    grad = torch.zeros((n, n, n), dtype=torch.float64, device=DEV)
+    ierr, _ = sol.solve(d["g"], d["b"], d["s"], w.sigma, x)
+    assert ierr.max() == 0
+    L, ierr = sol.adjoint(d["g"], -d["b"], d["s"], w.sigma, d["w"], x, y, grad)
+    assert ierr.max() == 0
+    Lo, go = ao.l_and_grad(w, list(range(w.nsys)), -w.rhs, weight, threshold=1e-13)
+    assert abs(L - Lo) <= 1e-10 * abs(Lo)
+    assert np.abs(grad.cpu().numpy() - go).max() <= 1e-9 * np.abs(go).max()
