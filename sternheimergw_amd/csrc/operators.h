@@ -138,6 +138,8 @@ class PwOperator : public Operator {
   // columns per plane that T and S need: the grid of the sphere's own
   // half-widths, at least ncs_ (nslot_ may count one half-width for all axes)
   int64_t box_cols_ = 0;
+  // one block per vector applies the operator (pwblock.h); else the batched kernels
+  bool block_ = false;
   DevBuf<int4> pk_info_, gr_info_;
   DevBuf<int32_t> pk_row_start_, pk_row_lo_, pk_row_cnt_;
   DevBuf<int32_t> gr_row_start_, gr_row_lo_, gr_row_cnt_;

@@ -12,8 +12,8 @@
 //                     with D = alpha_pv, the valence states of P_v.
 #include "operators.h"
 #include "ktimer.h"
-#include "lanes.h"
-#include "lines.h"
+#include "pwblock.h"
+#include "pwdev.h"
 #include "regfft.h"
 #include "splitfft.h"
 #include "tune.h"
@@ -63,39 +63,6 @@ __global__ __launch_bounds__(kBlock) void k_dense(int64_t n, const double2 *__re
 // ---------------------------------------------------------------------------
 // plane waves
 // ---------------------------------------------------------------------------
-struct PwDev {
-  int n1, n2, n3;
-  int M1, M2;           // column grid half widths; nc1 = 2M1+1, nc2 = 2M2+1
-  int nc1, nc2, nslot;
-  int64_t ld;
-  int nproj;
-  const double *vloc;          // [n3][n2][n1]
-  const double *vloc_zxy;      // [n3][n1][n2]: lanes of the x stage (one per y) read rows
-  const int32_t *npw;          // [ngroup]
-  const int32_t *col_start;    // [ngroup][nslot]
-  const int32_t *col_cnt;      // [ngroup][nslot]
-  const int32_t *sorted_idx;   // [ngroup][ld]
-  const int32_t *sorted_m3;    // [ngroup][ld] (reduced mod n3)
-  const int32_t *slot_of;      // [ngroup][ld]
-  const int32_t *m3_of;        // [ngroup][ld] (reduced mod n3)
-  const int32_t *col_lo;       // [ngroup][nslot] smallest m3 of the column
-  // column layout of the split z / plane transforms' T and S: ncs columns per
-  // plane; packed column j of group g is grid slot col_info[g][j].x (-1:
-  // none), with that column's count, start and lowest m3 in .y, .z, .w;
-  // row a of the grid holds columns m2 = row_lo .. row_lo + row_cnt - 1 at
-  // j = row_start[g][a] + m2 - row_lo (row_start[g][nc1]: the group's count)
-  int ncs;
-  const int4 *col_info;        // [ngroup][ncs]: (slot, col_cnt, col_start, col_lo)
-  const int32_t *row_start;    // [ngroup][nc1 + 1]
-  const int32_t *row_lo;       // [ngroup][nc1]
-  const int32_t *row_cnt;      // [ngroup][nc1]
-  const double *kin;           // [ngroup][ld]
-  const double2 *proj;         // [ngroup][nproj][ld]
-  const double *dcoef;         // [ngroup][nproj]
-  const double2 *tw1, *tw2, *tw3;  // e^{+2 pi i k/n}
-  double inv_nbox;
-};
-
 // One block per (plane z, vector v): pencil DFTs of one z-plane.
 // Output S[v][slot][z]: the plane's contribution to sum_z (...) before the
 // final z-transform.
@@ -1413,6 +1380,25 @@ __global__ __launch_bounds__(64 * W) void k_pw_reduce_split(
                                         reinterpret_cast<C *>(smem_d), relax, want, vlist);
 }
 
+// The whole application of one vector per block (pwblock.h)
+template <int N>
+__global__ __launch_bounds__(pwblock::threads(N)) void k_pw_block(
+    PwDev d, const double2 *__restrict__ in, int64_t sin, double2 *__restrict__ out, int64_t sout,
+    const double2 *__restrict__ sigma, const int32_t *__restrict__ active,
+    const int32_t *__restrict__ group, pwblock::Layout l) {
+  extern __shared__ double2 smem_d[];
+  const int v = blockIdx.x;
+  if (active && !active[v]) return;
+  const double2 *x = in + v * sin;
+  const int g = group ? group[v] : 0;
+  for (int e = threadIdx.x; e < d.ld; e += pwblock::threads(N)) smem_d[l.x + e] = x[e];
+  pwblock::load_tables<N>(d, g, smem_d, l);
+  __syncthreads();
+  double2 *o = out + v * sout;
+  pwblock::apply<N>(d, g, sigma[v], smem_d, l,
+                    [&](int e, double2 r) { o[e] = r; });
+}
+
 // planes per block and wavefronts per block of the split plane kernel where
 // no other shape is tried (mixed-precision batches): one plane on one
 // wavefront (on the 48 box the X stage in 1.5 rounds of 32 lane pairs, 13 KB
@@ -1665,6 +1651,16 @@ PwOperator::PwOperator(const PwDesc &desc) {
   tw_.upload(t1.data(), n1_);
   SGW_HIP(hipMemcpy(tw_.p + n1_, t2.data(), sizeof(double2) * n2_, hipMemcpyHostToDevice));
   SGW_HIP(hipMemcpy(tw_.p + n1_ + n2_, t3.data(), sizeof(double2) * n3_, hipMemcpyHostToDevice));
+  // The whole operator in one block where all planes of the box fit a CU's LDS
+  // at once (24^3 up to some 11 Ha).  1 vector, then 512: 28.4 and 45 us an
+  // application against 32.9 and 67 (6 Ha), 29.7 and 48 against 32.1 and 64
+  // (10 Ha).  Planes in two groups take 33.9 us against 33.2 (12 Ha), in three
+  // 39.8 against 33.4 (20 Ha); the 32^3 box 41 to 46 against 34, the 36^3 box
+  // 66 to 86 against 38.  The number of vectors has no part in the rule, so that
+  // a vector's result does not depend on its batch.
+  block_ = n1_ == 24 && n2_ == 24 && n3_ == 24 && columns_contiguous_ && fuse_stages_ &&
+           split_planes_ && band_planes_ &&
+           pwblock::layout(n1_, nc1_, ncs_, ld, nproj_).total * sizeof(double2) <= pwblock::kLds;
   SGW_HIP(hipDeviceSynchronize());
 }
 
@@ -1713,6 +1709,20 @@ void PwOperator::apply_work(hipStream_t st, int nvec, const double2 *in, int64_t
   const bool cubic = n1_ == n2_ && n2_ == n3_ && columns_contiguous_;
   const size_t lds_fft = sizeof(double2) * (nslot_ + (size_t)nc1_ * n1_);
   const dim3 gcol((unsigned)((nslot_ + 63) / 64), nvec);
+  if (block_ && fft_mode_ == 0) {
+    d.ncs = ncs_; d.col_info = pk_info_.p;
+    d.row_start = pk_row_start_.p; d.row_lo = pk_row_lo_.p; d.row_cnt = pk_row_cnt_.p;
+    const pwblock::Layout l = pwblock::layout(n1_, nc1_, ncs_, ld, nproj_);
+    const size_t lds = sizeof(double2) * (size_t)l.total;
+    KScope ks("pw_block", st, 2);
+    constexpr int NB = 24;
+    SGW_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(k_pw_block<NB>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    k_pw_block<NB><<<nvec, pwblock::threads(NB), lds, st>>>(d, in, in_stride, out, out_stride,
+                                                            d_sigma, d_active, d_group, l);
+    SGW_HIP(hipGetLastError());
+    return;
+  }
   const double2 *locv = nullptr;
   const int nchunk = (int)((ld + kChunk - 1) / kChunk);
   const int nred_x = (nproj_ * kVT + 63) / 64;
