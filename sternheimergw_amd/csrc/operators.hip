@@ -945,7 +945,8 @@ __global__ __launch_bounds__(64 * grad_waves(N), 3) void k_pw_plane_grad(
 // ---------------------------------------------------------------------------
 constexpr int kChunk = 64;
 constexpr int kVT = 16;
-constexpr int kAsmChunk = 64, kAsmThreads = 256;  // k_pw_assemble2 default block shape
+constexpr int kAsmThreads = 256;  // lanes of a k_pw_assemble2 block
+constexpr int kAsmBlocks = 640;   // blocks its widest shape has to fill
 
 // columns of nvec vectors of x and of as many of y (blockIdx.z) along z
 template <int N, int MB>
@@ -1021,11 +1022,13 @@ __device__ inline void becp_reduce_body(const PwDev &d, const int32_t *__restric
 }
 
 // part[((g*tiles + vt)*nchunk + chunk)][p][vl] = sum_{i in chunk} conj(proj_p(i)) x_v(i)
+// for p0 <= p < pe: all projectors, or at most 16 of them
 __device__ inline void becp_body(const PwDev &d, const double2 *__restrict__ in, int64_t sin,
                                  const int32_t *__restrict__ active,
                                  const int32_t *__restrict__ gvec,
                                  const int32_t *__restrict__ gcnt, int maxper, int tiles,
-                                 int nchunk, double2 *__restrict__ part, int chunk, int g, int vt);
+                                 int nchunk, double2 *__restrict__ part, int chunk, int g, int vt,
+                                 int p0, int pe);
 
 __global__ __launch_bounds__(256) void k_pw_becp(PwDev d, const double2 *__restrict__ in,
                                                  int64_t sin, const int32_t *__restrict__ active,
@@ -1034,14 +1037,15 @@ __global__ __launch_bounds__(256) void k_pw_becp(PwDev d, const double2 *__restr
                                                  int tiles, int nchunk,
                                                  double2 *__restrict__ part) {
   becp_body(d, in, sin, active, gvec, gcnt, maxper, tiles, nchunk, part, blockIdx.x, blockIdx.y,
-            blockIdx.z);
+            blockIdx.z, 0, d.nproj);
 }
 
 __device__ inline void becp_body(const PwDev &d, const double2 *__restrict__ in, int64_t sin,
                                  const int32_t *__restrict__ active,
                                  const int32_t *__restrict__ gvec,
                                  const int32_t *__restrict__ gcnt, int maxper, int tiles,
-                                 int nchunk, double2 *__restrict__ part, int chunk, int g, int vt) {
+                                 int nchunk, double2 *__restrict__ part, int chunk, int g, int vt,
+                                 int p0, int pe) {
   const int cnt = gcnt[g], v0 = vt * kVT;
   const int npw = d.npw[g], i0 = chunk * kChunk;
   if (v0 >= cnt || i0 >= npw) return;
@@ -1066,11 +1070,11 @@ __device__ inline void becp_body(const PwDev &d, const double2 *__restrict__ in,
   const double2 *pg = d.proj + (int64_t)g * nproj * d.ld + i0;
   double2 *pout = part + (((int64_t)g * tiles + vt) * nchunk + chunk) * nproj * kVT;
   const int npb = (nproj + kPB - 1) / kPB;
-  const bool few = nproj <= 16;
+  const bool few = pe - p0 <= 16;
   double2 next[4];
   auto load = [&](int p, int i) {
-    const double2 q = pg[(int64_t)min(p, nproj - 1) * d.ld + min(i, lim - 1)];
-    const bool in = p < nproj && i < lim;
+    const double2 q = pg[(int64_t)min(p, pe - 1) * d.ld + min(i, lim - 1)];
+    const bool in = p < pe && i < lim;
     return mk(in ? q.x : 0.0, in ? q.y : 0.0);
   };
   auto fetch = [&](int stage) {  // stage = projector block, then plane-wave block
@@ -1080,7 +1084,7 @@ __device__ inline void becp_body(const PwDev &d, const double2 *__restrict__ in,
   };
   if (few) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) next[r] = load(wv + 4 * r, lane);
+    for (int r = 0; r < 4; ++r) next[r] = load(p0 + wv + 4 * r, lane);
   } else {
     fetch(0);
   }
@@ -1100,7 +1104,7 @@ __device__ inline void becp_body(const PwDev &d, const double2 *__restrict__ in,
     const int p = tid / kVT, vl = tid % kVT;
     double2 acc = mk(0, 0);
     for (int i = 0; i < lim; ++i) cmacc(acc, rows[p * (kChunk + 1) + i], xs[vl][i]);
-    if (p < nproj) pout[p * kVT + vl] = acc;
+    if (p0 + p < pe) pout[(p0 + p) * kVT + vl] = acc;
     return;
   }
   const int tp = 16 * wv + (lane >> 3), tv = lane & 7;
@@ -1167,12 +1171,12 @@ __global__ __launch_bounds__(NT) void k_pw_assemble2(
   const int i = threadIdx.x % CH, vq = threadIdx.x / CH;
   const int64_t e = (int64_t)i0 + i;
   const bool inside = e < npw;
-  // kAhead projector values are loaded together, the first from before the
-  // overlaps are in LDS.  The loads are unconditional (past the last projector
+  // kAhead projector values are loaded together, the first before the overlaps
+  // are in LDS.  One vector to a thread leaves registers for 16.  The loads are unconditional (past the last projector
   // they repeat it): under a condition each would be waited for by itself.
   // A second set in flight (16 + 16) costs a wavefront per SIMD: 18.4 us per
   // launch of the streamed 48^3 solve against 15.0.
-  constexpr int kAhead = 8;
+  constexpr int kAhead = CH == 16 ? 16 : 8;
   const double2 *pg = d.proj + (int64_t)g * nproj * d.ld + (inside ? e : 0);
   double2 pv[kAhead];
   auto fetch = [&](int p0) {
@@ -1304,20 +1308,23 @@ template <int N, bool SPLIT, int MB, typename C = double2, bool RL = false>
 __global__ __launch_bounds__(256) void k_pw_becp_zinv(
     PwDev d, const double2 *__restrict__ in, int64_t sin, const int32_t *__restrict__ group,
     const int32_t *__restrict__ active, const int32_t *__restrict__ gvec,
-    const int32_t *__restrict__ gcnt, int maxper, int tiles, int nchunk, int ngroup,
+    const int32_t *__restrict__ gcnt, int maxper, int tiles, int nchunk, int ngroup, int psplit,
     double2 *__restrict__ part, C *__restrict__ T, int nvec,
     const int32_t *__restrict__ relax = nullptr, int want = 0,
     int32_t *__restrict__ vlist = nullptr) {
   // with a list to build, block 0 builds it (first, so that its serial
   // scan does not trail the launch) and the others shift down by one
-  const int nbecp = nchunk * ngroup * tiles, b = (int)blockIdx.x - (vlist ? 1 : 0);
+  // psplit blocks take 16 projectors each of a chunk and tile, or one takes all
+  const int nbecp = nchunk * ngroup * tiles * psplit, b = (int)blockIdx.x - (vlist ? 1 : 0);
   if (b < 0) {
     vlist_body(nvec, active, vlist);
     return;
   }
   if (b < nbecp) {
-    becp_body(d, in, sin, active, gvec, gcnt, maxper, tiles, nchunk, part, b % nchunk,
-              (b / nchunk) % ngroup, b / (nchunk * ngroup));
+    const int ps = b % psplit, c = b / psplit;
+    becp_body(d, in, sin, active, gvec, gcnt, maxper, tiles, nchunk, part, c % nchunk,
+              (c / nchunk) % ngroup, c / (nchunk * ngroup), 16 * ps,
+              psplit > 1 ? min(d.nproj, 16 * ps + 16) : d.nproj);
     return;
   }
   constexpr int kCols = SPLIT ? 32 : 64;  // columns per 64-lane group
@@ -1749,7 +1756,15 @@ void PwOperator::apply_work(hipStream_t st, int nvec, const double2 *in, int64_t
     if (fused) {
       // no projectors: the part counts are zero and only the transforms run
       const int tiles = nproj_ > 0 ? wk.plan_tiles : 0;
-      const int64_t nbecp = (int64_t)nchunk * ngroup_ * tiles;
+      // Few chunks and tiles leave the chip idle behind each block's stages: 16
+      // projectors to a block then, in one stage.  48^3 (48 projectors, 26
+      // chunks of 64 plane waves): 16 vectors 7.0 us against 9.6, 64 vectors
+      // 10.4 against 13.6, 128 vectors (624 blocks) 16.3 against 13.3; 36^3 (26
+      // projectors, 10 chunks): 256 vectors 9.8 against 12.8.
+      const int64_t nsum = (int64_t)nchunk * ngroup_ * tiles;
+      const int nsplit = (nproj_ + 15) / 16;
+      const int psplit = nsum * nsplit <= 512 ? std::max(nsplit, 1) : 1;
+      const int64_t nbecp = nsum * psplit;
       // fft_mode_: 0 FP64, 1 FP32, 2 per vector from the relax flags.  With
       // both precisions the FP64 instances carry the projector sums and the
       // FP32 ones (tiles 0) the transforms of the relaxed vectors only.  The
@@ -1762,7 +1777,7 @@ void PwOperator::apply_work(hipStream_t st, int nvec, const double2 *in, int64_t
       };
       const bool run64 = fft_mode_ != 1, run32 = fft_mode_ != 0;
       const int tiles32 = run64 ? 0 : tiles;
-      const int64_t nbecp32 = (int64_t)nchunk * ngroup_ * tiles32;
+      const int64_t nbecp32 = (int64_t)nchunk * ngroup_ * tiles32 * psplit;
       float2 *T32 = reinterpret_cast<float2 *>(wk.T), *S32 = reinterpret_cast<float2 *>(wk.S);
       // z transforms split over lane pairs: 32 columns per 64 lanes
       const bool zsplit = split_planes_;
@@ -1794,18 +1809,18 @@ void PwOperator::apply_work(hipStream_t st, int nvec, const double2 *in, int64_t
                 k_pw_becp_zinv<NB, true, decltype(mb)::value, double2, decltype(rlt)::value>
                     <<<(unsigned)(nbecp + nzinv + (vl64 ? 1 : 0)), 256, 0, st>>>(
                         d, in, in_stride, d_group, d_active, wk.plan_vec, wk.plan_cnt,
-                        wk.plan_max, tiles, nchunk, ngroup_, wk.part, wk.T, nvec, rl, 0, vl64);
+                        wk.plan_max, tiles, nchunk, ngroup_, psplit, wk.part, wk.T, nvec, rl, 0, vl64);
               });
             if (run32)
               k_pw_becp_zinv<NB, true, decltype(mb)::value, float2, true>
                   <<<(unsigned)(nbecp32 + nzinv + (vl32 ? 1 : 0)), 256, 0, st>>>(
                       d, in, in_stride, d_group, d_active, wk.plan_vec, wk.plan_cnt, wk.plan_max,
-                      tiles32, nchunk, ngroup_, wk.part, T32, nvec, rl, 1, vl32);
+                      tiles32, nchunk, ngroup_, psplit, wk.part, T32, nvec, rl, 1, vl32);
           });
         else
           k_pw_becp_zinv<NB, false, -1><<<(unsigned)(nbecp + nzinv), 256, 0, st>>>(
               d, in, in_stride, d_group, d_active, wk.plan_vec, wk.plan_cnt, wk.plan_max, tiles,
-              nchunk, ngroup_, wk.part, wk.T, nvec);
+              nchunk, ngroup_, psplit, wk.part, wk.T, nvec);
       }
       {
         KScope ks("pw_reduce_plane", st, 2);
@@ -1964,12 +1979,16 @@ void PwOperator::apply_work(hipStream_t st, int nvec, const double2 *in, int64_t
   {
     const size_t lds_asm = sizeof(double2) * (size_t)nproj_ * kVT;
     KScope ks("pw_assemble", st, 2);
-    // 64 plane waves x 4 vector groups per 256-lane block by default: on the
-    // 48^3 batch 21.9 us per 512 vectors against 26.4 with 32 plane waves x 8
-    // groups and 33.2 with 16 x 16, and the one the autotuner keeps there;
-    // the autotuner tries 32 and 16 as well for each size class of the batch
-    // (not when the output overwrites the input, which a second launch would
-    // read)
+    // 64 plane waves x 4 vector groups, 32 x 8 or 16 x 16 to a block.  Wide
+    // blocks read a projector value once for four vectors; narrow ones fill the
+    // chip for a small batch and have fewer products in a row.  The widest with
+    // kAsmBlocks blocks goes first: 48^3 (48 projectors, 26 chunks of 64) 512
+    // vectors 21.0 / 23.9 / 28.8 us, 256 vectors 16.0 / 15.2 / 17.7, 64 vectors
+    // 14.4 / 10.9 / 9.6 (8.7 with 16 values together), 16 vectors 12.6 / 9.1 / 7.8;
+    // 36^3 (26 projectors, 10 chunks) 512 vectors 12.6 / 10.8 / 11.2, 256 vectors
+    // 11.4 / 9.2 / 8.8.  The autotuner tries the others for each size class of
+    // the batch (not when the output overwrites the input, which a second
+    // launch would read)
     constexpr int NT = kAsmThreads;
     auto launch_asm = [&](auto chunk) {
       constexpr int CH = decltype(chunk)::value;
@@ -1978,13 +1997,18 @@ void PwOperator::apply_work(hipStream_t st, int nvec, const double2 *in, int64_t
                                               wk.plan_vec, wk.plan_cnt, wk.plan_max,
                                               wk.plan_tiles, nchunk, wk.becp, wk.S, locv);
     };
+    const int64_t per = (int64_t)ngroup_ * wk.plan_tiles;
+    const int first = (ld + 63) / 64 * per >= kAsmBlocks   ? 0
+                      : (ld + 31) / 32 * per >= kAsmBlocks ? 1
+                                                           : 2;
     const bool disjoint = out + (int64_t)(nvec - 1) * out_stride + ld <= in ||
                           in + (int64_t)(nvec - 1) * in_stride + ld <= out;
     const std::string key = "assemble/n" + std::to_string(size_class(nvec)) + "/g" +
                             std::to_string(ngroup_) + "/p" + std::to_string(nproj_);
     autotune(key, disjoint ? 3 : 1, st, [&](int c) {
-      if (c == 0) launch_asm(std::integral_constant<int, kAsmChunk>{});
-      else if (c == 1) launch_asm(std::integral_constant<int, 32>{});
+      const int shape = (first + c) % 3;
+      if (shape == 0) launch_asm(std::integral_constant<int, 64>{});
+      else if (shape == 1) launch_asm(std::integral_constant<int, 32>{});
       else launch_asm(std::integral_constant<int, 16>{});
     });
   }

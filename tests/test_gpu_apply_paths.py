@@ -73,8 +73,9 @@ def _cell(n, ecut, nbeta, nocc, ngroup, gap=False):
     (24, 6.0, 8, 4, 5, False),    # one block, 4 threads' sums to a plane wave
     (24, 8.0, 60, 5, 3, False),   # 2 threads' sums
     (24, 10.0, 17, 0, 5, False),  # one thread's sum
-    (24, 10.0, 1800, 10, 1, False),  # the projectors leave no room
-    (24, 12.0, 17, 0, 5, False),  # the planes leave none
+    (24, 10.0, 290, 10, 1, False),
+    (24, 12.0, 17, 0, 5, False),  # the planes leave no room
+    (24, 12.0, 290, 10, 1, False),
     (24, 20.0, 8, 8, 2, False),
     (24, 30.0, 8, 4, 2, False),
     (24, 6.0, 8, 4, 2, True),
