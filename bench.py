@@ -341,7 +341,8 @@ def run_sigma_real(args):
     _lib.check(L.sgw_kernel_timing_query(b"sigma_prod", ctypes.byref(ms), ctypes.byref(cnt)))
     _lib.check(L.sgw_kernel_timing(0))
     nr = n ** 3
-    bytes_per = 16.0 * (4 * ng * nr + 7 * nr * nr)
+    # the rows' transforms out and back through memory, G read once
+    bytes_per = 16.0 * (4 * ng * nr + nr * nr)
     t_prod = ms.value / 1e3 / max(cnt.value, 1)
     achieved = bytes_per / t_prod / 1e9
     prods = ngreen * nsig * args.steps
@@ -355,7 +356,7 @@ def run_sigma_real(args):
         "data": "synthetic (random G(r,r') and W(G,G',i w) on the device)",
         "config": {"workload": "sigma-real-24^3: N_G 1500, Pade W (4 points), 8 Green x 2 Sigma "
                                "frequencies per step", "n": n, "num_g": ng},
-        "roofline": {"kernel": "sigma_prod (box FFT passes + index maps + product)",
+        "roofline": {"kernel": "sigma_prod (sphere-to-box FFTs and the product, a box per block)",
                      "bound": "hbm", "achieved": round(achieved, 1), "peak": 8000.0,
                      "unit": "GB/s", "frac": round(achieved / 8000.0, 4), "traffic": None,
                      "algorithmic_bytes_per_launch": bytes_per, "launches": cnt.value,
