@@ -1058,7 +1058,7 @@ __device__ inline void becp_body(const PwDev &d, const double2 *__restrict__ in,
   // their 16 x 16 (projector, vector) sums, one operand read from LDS a product
   // where one sum per lane takes two; the plane waves come 16 at a time.  On
   // the 48^3 box (48 projectors, 512 slots streamed) with the z transforms
-  // beside it 16.8 us a launch against 19.6 with one sum to a lane.
+  // beside it 18.1 us a launch against 19.6 with one sum to a lane.
   // Loads are unconditional, their places clamped: under a condition each is
   // waited for by itself.
   constexpr int kIB = 16, kPB = 64;
