@@ -52,7 +52,10 @@ template <int H> __device__ inline double2 wsum2(const double2 (&v)[H]) {
 __device__ inline uint32_t gballot(bool c) {
   return (uint32_t)(__ballot(c) >> (threadIdx.x & 32));
 }
-__device__ inline double cabs2a(double2 a) { return a.x * a.x + a.y * a.y; }
+// the form is spelled out: a weight vector is fixed up to a phase, which comes
+// from the rotations of rounding-level pairs, so that the last bit of a norm
+// shows in the coefficients
+__device__ inline double cabs2a(double2 a) { return fma(a.x, a.x, a.y * a.y); }
 __device__ inline double cabsa(double2 a) { return hypot(a.x, a.y); }
 
 __device__ inline uint64_t below(int l) { return l == 0 ? 0ull : (~0ull >> (64 - l)); }
