@@ -103,8 +103,11 @@ __host__ __device__ inline int aaa_lds(int M, int mcap) { return (M + mcap + 4) 
 // Bound: the dependent FP64 chains of the Jacobi pairs.  H mesh points and
 // matrix rows to a lane; two elements share a wavefront, and the group sums
 // are vector instructions (lanes.h), so the rows of a pair wait for no LDS
-// permute.  400 x 400 elements, 35 points, at most 11 support points: 18.2 ms,
-// against 42.4 with one wavefront per element and LDS-permute sums.
+// permute.  400 x 400 elements, 35 points, at most 11 support points: 16.3 ms,
+// against 42.4 with one wavefront per element and LDS-permute sums.  Zeros
+// are written out where a value or zero is chosen: a named one makes the choice
+// one of addresses, for which the compiler copies the whole mesh to private
+// memory (1 312 bytes a lane, 18.2 ms).
 template <int H>
 __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh mesh, double thres,
                                                   int model, int max_point, int mcap,
@@ -120,7 +123,6 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
   double2 *val = pos + mcap;
   double2 *wgt = val + mcap;
   double2 *lam = wgt + mcap;
-  const double2 zero = mk(0.0, 0.0);
   const uint64_t all = M == 64 ? ~0ull : (1ull << M) - 1;
   double2 zl[H], fl[H], fit[H];
   bool pt[H], sup[H];
@@ -130,8 +132,8 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
     const int i = l + kGrp * h;
     pt[h] = i < M;
     sup[h] = false;
-    zl[h] = pt[h] ? mesh.z[i] : zero;
-    fl[h] = pt[h] ? w[(int64_t)mesh.src[i] * ne + e] : zero;
+    zl[h] = pt[h] ? mesh.z[i] : mk(0.0, 0.0);
+    fl[h] = pt[h] ? w[(int64_t)mesh.src[i] * ne + e] : mk(0.0, 0.0);
     d[h] = pt[h] ? cabsa(fl[h]) : 0.0;
   }
   // setup_work_type (:119-148)
@@ -191,7 +193,7 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
     __syncwarp();
     auto column = [&](int c, double2 (&a)[H]) {
 #pragma unroll
-      for (int h = 0; h < H; ++h) a[h] = l + kGrp * h < nrows ? A[c * M + l + kGrp * h] : zero;
+      for (int h = 0; h < H; ++h) a[h] = l + kGrp * h < nrows ? A[c * M + l + kGrp * h] : mk(0.0, 0.0);
     };
     auto norm2 = [&](const double2 (&a)[H]) {
       double s[H];
@@ -208,7 +210,7 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
           // column p stays in registers over its pairs
           double2 ap[H], aq[H];
           column(p, ap);
-          double2 vp = l < m ? V[p * mcap + l] : zero;
+          double2 vp = l < m ? V[p * mcap + l] : mk(0.0, 0.0);
           double al = norm2(ap);
           bool turned = false;
           for (int q = p + 1; q < m; ++q) {
@@ -217,7 +219,7 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
             double2 gh[H];
 #pragma unroll
             for (int h = 0; h < H; ++h) {
-              gh[h] = zero;
+              gh[h] = mk(0.0, 0.0);
               cmacc(gh[h], ap[h], aq[h]);
             }
             const double2 gm = wsum2<H>(gh);
@@ -277,7 +279,7 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
 #pragma unroll
     for (int h = 0; h < H; ++h)
       if (pt[h] && !sup[h]) {
-        double2 num = zero, den = zero;
+        double2 num = mk(0.0, 0.0), den = mk(0.0, 0.0);
         for (int c = 0; c < m; ++c) {
           const double2 cc = cauchy(zl[h], pos[c]);
           num = cadd(num, cmul(cc, cmul(wgt[c], val[c])));
@@ -299,7 +301,7 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
   if (model == 4) {
     const int mmax = max_point;
     for (int s = l; s < M; s += kGrp) {
-      double2 v = zero;
+      double2 v = mk(0.0, 0.0);
       if (s < m) v = pos[s];
       else if (s >= mmax && s < mmax + m) v = val[s - mmax];
       else if (s >= 2 * mmax && s < 2 * mmax + m) v = wgt[s - 2 * mmax];
@@ -310,7 +312,7 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
   // model 5: poles (zeros of the denominator) by Aberth-Ehrlich, then the
   // residues of calculate_residual (:458-500) and pole_correction's filter
   const int nr = m - 1;
-  const double2 mine[1] = {l < m ? pos[l] : zero};
+  const double2 mine[1] = {l < m ? pos[l] : mk(0.0, 0.0)};
   double2 cen = wsum2<1>(mine);
   cen = mk(cen.x / m, cen.y / m);
   double rad = lanes::max<kGrp>(l < m ? cabsa(csub(pos[l], cen)) : 0.0);
