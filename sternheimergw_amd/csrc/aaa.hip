@@ -30,6 +30,7 @@ constexpr double kDblEpsA = 2.220446049250313e-16;
 constexpr int kSweeps = 40, kAberthIters = 500;
 
 constexpr int kGrp = 32;                                // lanes per element
+constexpr size_t kLdsCu = 160 * 1024;                   // LDS bytes of a CU
 
 // sums and extrema over the mesh points or matrix rows of an element, H to a
 // lane; the order is that of a 64-lane butterfly (lane l and l + 32 first)
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
                                                   double2 *__restrict__ w,
                                                   int32_t *__restrict__ status) {
   extern __shared__ double2 aaa_smem[];
-  const int64_t e = (int64_t)blockIdx.x * 2 + threadIdx.x / kGrp;
+  const int64_t e = (int64_t)blockIdx.x * (blockDim.x / kGrp) + threadIdx.x / kGrp;
   const int l = threadIdx.x % kGrp;
   if (e >= ne) return;
   double2 *A = aaa_smem + (size_t)(threadIdx.x / kGrp) * aaa_lds(M, mcap);
@@ -405,15 +406,20 @@ void aaa_coeffs(int model, double thres, int64_t ne, int nfreq, const double2 *z
   // unique)
   const int max_point = model == 4 ? nfreq / 3 : nfreq;
   const int mcap = model == 4 ? nfreq / 3 : nfreq / 2;
-  const size_t lds = 2 * sizeof(double2) * (size_t)aaa_lds(nfreq, mcap);  // <= 102400
+  // Two elements share a wavefront while a CU's LDS holds more of them than its
+  // SIMDs hold wavefronts (16); where it holds fewer, each has a wavefront of its
+  // own, and a CU takes an odd number of them too.  A wavefront each against two
+  // together: model 4 at 32 points (22 to a CU) 20.0 ms against 19.3, at 36
+  // points (16) 38.7 against 42.2, at 64 (5) 113 against 187; model 5 at 24 points
+  // (21) 37.4 against 35.8, at 36 (10) 180 against 240, at 64 (3) 633 against 1 415.
+  const size_t one = sizeof(double2) * (size_t)aaa_lds(nfreq, mcap);  // <= 51200
+  const int per = kLdsCu / one > 16 ? 2 : 1;
+  const size_t lds = per * one;
   DevBuf<int32_t> status(2);
   SGW_HIP(hipMemsetAsync(status.p, 0, 2 * sizeof(int32_t), st));
   auto *kern = nfreq <= kGrp ? k_aaa_coeffs<1> : k_aaa_coeffs<2>;
-  if (lds > 64 * 1024)
-    SGW_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-  kern<<<(unsigned)((ne + 1) / 2), 64, lds, st>>>(ne, nfreq, mesh, thres, model, max_point, mcap,
-                                                  d_w, status.p);
+  kern<<<(unsigned)((ne + per - 1) / per), kGrp * per, lds, st>>>(
+      ne, nfreq, mesh, thres, model, max_point, mcap, d_w, status.p);
   SGW_HIP(hipGetLastError());
   int32_t h[2] = {0, 0};
   SGW_HIP(hipMemcpyAsync(h, status.p, sizeof(h), hipMemcpyDeviceToHost, st));
