@@ -450,7 +450,9 @@ int sgw_green_assemble(int32_t nfreq, int32_t n, int32_t n_p, int32_t nrow,
  * (SGW_E_STATE, the element's slices NaN): more relevant poles than
  * nfreq / 2 (the reference's errore), or an SGW_AAA_POLE element that is
  * not converged at nfreq / 2 support points (the Loewner submatrix would
- * have more columns than rows and no unique null vector). */
+ * have more columns than rows and no unique null vector) or has a NaN
+ * sample.  SGW_AAA_APPROX leaves an element with a NaN sample as NaN in all
+ * slices. */
 int sgw_analytic_coeff(int32_t model, double thres, int32_t num_g, int32_t nfreq,
                        const sgw_complex *h_z, const int32_t *h_src, sgw_complex *d_w,
                        void *stream);

@@ -98,7 +98,8 @@ __host__ __device__ inline int aaa_lds(int M, int mcap) { return (M + mcap + 4) 
 
 // model 4: slices [pos (mmax), val (mmax), wgt (mmax), 0...], mmax = max_point;
 // model 5: [poles, 0..., residues, 0...] in halves of N / 2.
-// status[0] = 1: a model-5 element needed more than mcap support points;
+// status[0] = 1: a model-5 element needed more than mcap support points, or has
+// NaN samples;
 // status[1] = 1: more relevant poles than N / 2 (pole_correction's error)
 //
 // Bound: the dependent FP64 chains of the Jacobi pairs.  H mesh points and
@@ -143,6 +144,7 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
 #pragma unroll
   for (int h = 0; h < H; ++h) fit[h] = mk(sumf.x / M, sumf.y / M);
   int m = 0;
+  bool lost = false;
   const int mp = max_point;
   for (;;) {
     // update_support_point (:178-187): the first point of largest |f - fit|
@@ -167,6 +169,13 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
     smask &= all;
     const uint64_t rmask = ~smask & all;
     const int nrows = M - m;
+    // a NaN among the samples leaves no point of largest error (none, or one
+    // past the mesh, or a support point again)
+    lost = __popcll(smask) != m;
+    if (lost) {
+      if (l == 0 && model == 5) status[0] = 1;
+      break;
+    }
     if (m > mcap) {  // the device keeps at most mcap support points
       if (l == 0) status[0] = 1;
       break;
@@ -295,7 +304,7 @@ __global__ __launch_bounds__(64) void k_aaa_coeffs(int64_t ne, int M, AaaMesh me
     if (wmax<H>(d) == 0.0 || m >= mp) break;
   }
   __syncwarp();
-  if (m > mcap) {  // flagged: the coefficients are left as NaN
+  if (lost || m > mcap) {  // the coefficients are left as NaN
     for (int s = l; s < M; s += kGrp) w[(int64_t)s * ne + e] = mk(NAN, NAN);
     return;
   }
@@ -425,7 +434,8 @@ void aaa_coeffs(int model, double thres, int64_t ne, int nfreq, const double2 *z
   SGW_HIP(hipMemcpyAsync(h, status.p, sizeof(h), hipMemcpyDeviceToHost, st));
   SGW_HIP(hipStreamSynchronize(st));
   SGW_REQUIRE(h[0] == 0, SGW_E_STATE,
-              "aaa: an element needs more than N/2 support points (its coefficients are NaN)");
+              "aaa: an element needs more than N/2 support points, or has NaN samples (its "
+              "coefficients are NaN)");
   SGW_REQUIRE(h[1] == 0, SGW_E_STATE,
               "aaa: two many relevant poles, try reducing the coulomb threshold or increasing "
               "the number of frequencies (the element's coefficients are NaN)");

@@ -66,3 +66,31 @@ def test_coefficients_keep_their_bits(n, model):
         | np.uint64(1)
     sums = (words * odd).sum(1, dtype=np.uint64)
     assert np.array_equal(sums, gold[f"{n}_{model}"]), np.flatnonzero(sums != gold[f"{n}_{model}"])
+
+
+@pytest.mark.parametrize("n", [3, 12, 32, 35, 64])
+def test_nan_sample_gives_nan_coefficients(n):
+    """An element with a NaN among its samples has no largest error to place a
+    support point at: all its coefficients are NaN (SGW_AAA_POLE, which needs
+    the fit to converge, refuses the call), and no other element changes."""
+    print(f"AAA with NaN samples n={n}", flush=True)
+    z, w = _elements(n, 5)
+    bad = {(0, 0): [0], (1, 3): [n // 2], (2, 2): [n - 1], (4, 4): list(range(n))}
+    wn = w.copy()
+    for (c, r), rows in bad.items():
+        wn[rows, c, r] = complex(np.nan, 1.0)
+    plain, d = torch.from_numpy(w).to(DEV), torch.from_numpy(wn).to(DEV)
+    # what earlier kernels leave in LDS is no number of these elements
+    junk = torch.full((n, 40, 40), 3.25 + 0.5j, dtype=torch.complex128, device=DEV)
+    sigma_real.ScreenedCoulomb(junk, z, _lib.AAA_APPROX, thres=1e-10)
+    sigma_real.ScreenedCoulomb(plain, z, _lib.AAA_APPROX, thres=1e-10)
+    sigma_real.ScreenedCoulomb(d, z, _lib.AAA_APPROX, thres=1e-10)
+    got, want = d.cpu().numpy(), plain.cpu().numpy()
+    for c in range(5):
+        for r in range(5):
+            if (c, r) in bad:
+                assert np.isnan(got[:, c, r]).all(), (c, r)
+            else:
+                assert np.array_equal(got[:, c, r], want[:, c, r]), (c, r)
+    with pytest.raises(_lib.SgwError):
+        sigma_real.ScreenedCoulomb(torch.from_numpy(wn).to(DEV), z, _lib.AAA_POLE, thres=1e-10)
