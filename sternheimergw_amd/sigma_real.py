@@ -106,6 +106,20 @@ def sigma_prod(grid: CorrGrid, grid_p: CorrGrid, omega_cell: float, alpha, d_gre
     return d_array
 
 
+def _green_offsets(d_green_r, num_green, size):
+    """Where the first num_green matrices of `size` elements start in the stack
+    d_green_r, in elements: the library takes offsets without an end, so the
+    stack has to hold them."""
+    import torch
+    if d_green_r.shape[0] < num_green:
+        raise IndexError(f"{num_green} Green's functions needed, the stack holds "
+                         f"{d_green_r.shape[0]}")
+    one = d_green_r[0]
+    if one.dtype != torch.complex128 or one.numel() < size or not one.is_contiguous():
+        raise ValueError("each G(r, r') must be a contiguous complex128 (nr_p, nr) matrix")
+    return np.arange(num_green, dtype=np.int64) * d_green_r.stride(0)
+
+
 def sigma_correlation(grid: CorrGrid, grid_p: CorrGrid, omega_cell: float, alpha, mu, coul,
                       weight, sigma_freq, d_green_r, w: ScreenedCoulomb, gmap=None, gmap_p=None):
     """Sigma_c(G, G'; omega_sigma) of sigma.f90:653-745.  d_green_r:
@@ -124,6 +138,7 @@ def sigma_correlation(grid: CorrGrid, grid_p: CorrGrid, omega_cell: float, alpha
     sigma = torch.zeros((freq_sigma.size, grid_p.num_g, grid.num_g), dtype=torch.complex128,
                         device=dev)
     nterm = freq_sigma.size * freq_green.size
+    offset = _green_offsets(d_green_r, freq_green.size, grid_p.nr * grid.nr)
     freq = np.empty(nterm, dtype=np.complex128)
     alphas = np.empty(nterm, dtype=np.complex128)
     igs = np.tile(np.arange(freq_green.size, dtype=np.int32), freq_sigma.size)
@@ -134,7 +149,7 @@ def sigma_correlation(grid: CorrGrid, grid_p: CorrGrid, omega_cell: float, alpha
             fc = np.conj(fc)
         freq[t] = w.symmetrize(fc)                                   # :714
         alphas[t] = alpha * weight[igs[t] % num_coul]                # :722, :725
-    at = igs.astype(np.int64) * d_green_r.stride(0)
+    at = offset[igs]
     lib = _lib.lib()
     need = lib.sgw_sigma_correlation_workspace(grid.n, grid_p.n, grid.num_g, grid_p.num_g)
     work = torch.empty(max(need, 1), dtype=torch.uint8, device=dev)
