@@ -138,6 +138,8 @@ def sigma_correlation(grid: CorrGrid, grid_p: CorrGrid, omega_cell: float, alpha
     sigma = torch.zeros((freq_sigma.size, grid_p.num_g, grid.num_g), dtype=torch.complex128,
                         device=dev)
     nterm = freq_sigma.size * freq_green.size
+    if nterm == 0:
+        return sigma
     offset = _green_offsets(d_green_r, freq_green.size, grid_p.nr * grid.nr)
     freq = np.empty(nterm, dtype=np.complex128)
     alphas = np.empty(nterm, dtype=np.complex128)

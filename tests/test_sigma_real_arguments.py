@@ -58,3 +58,10 @@ def test_strided_stack_is_taken(monkeypatch):
     with pytest.raises(_Reached):
         _setup(monkeypatch)(_stack(8, 6, 8)[::2])
     assert list(sigma_real._green_offsets(_stack(8, 6, 8)[::2], 4, 48)) == [0, 96, 192, 288]
+
+
+@pytest.mark.parametrize("coul,sigma_freq", [((), (0.0, 0.2)), ((0.1j,), ()), ((), ())])
+def test_no_terms_is_a_zero_sigma(monkeypatch, coul, sigma_freq):
+    call = _setup(monkeypatch)
+    out = call(_stack(2 * len(coul), 6, 8), coul, sigma_freq)
+    assert out.shape == (len(sigma_freq), 2, 3) and not out.any()
