@@ -459,8 +459,9 @@ int sgw_analytic_coeff(int32_t model, double thres, int32_t num_g, int32_t nfreq
 
 /* analytic_eval (analytic.f90:211-348): out(nr, nr_p) = 0, then
  * out(r, c) = W_model(freq; coeff(gmap[r], gmap_p[c], :)) for r < num_g,
- * c < num_g_p (gmap: gmapsym, gmap_p: gmapsym(fft_map), 0-based).  freq is
- * the symmetrised output frequency (freq_in%symmetrize).  Robust Pade
+ * c < num_g_p (gmap: gmapsym, gmap_p: gmapsym(fft_map), 0-based; num_g and
+ * num_g_p entries, NaN where one is outside W's num_gc).  freq is the
+ * symmetrised output frequency (freq_in%symmetrize).  Robust Pade
  * (pade_eval_robust, pade_robust.f90:37-86) reads the degrees from the first
  * two slices (h_z may be NULL); an element whose degrees do not fit the
  * nfreq slices evaluates to NaN.  AAA (aaa_approx_eval, aaa_pole_eval,

@@ -33,6 +33,17 @@ def _cplx(z):
     return _lib.sgw_complex(float(np.real(z)), float(np.imag(z)))
 
 
+def _map(d_map, num_g):
+    """The map of num_g G vectors to W's as the library reads it: one 32-bit
+    entry for each of them.  Behind the end of a shorter map no element exists
+    (-1, which evaluates to NaN)."""
+    import torch
+    d_map = d_map.to(torch.int32).contiguous()
+    if d_map.numel() < num_g:
+        d_map = torch.nn.functional.pad(d_map.reshape(-1), (0, num_g - d_map.numel()), value=-1)
+    return d_map
+
+
 def freqbins_symm(solver, symm):
     """The symmetrised mesh of freqbins.f90:333-425 and, for every point,
     the solver frequency whose W it carries."""
@@ -87,7 +98,9 @@ class ScreenedCoulomb:
         return freq ** 2 if self.symm == SQUARE_SYMMETRY else freq
 
     def eval_into(self, freq, grid: CorrGrid, grid_p: CorrGrid, d_gmap, d_gmap_p, out):
-        """analytic_eval (analytic.f90:211-348) into out (nr_p, nr)."""
+        """analytic_eval (analytic.f90:211-348) into out (nr_p, nr); NaN where a
+        map has no entry or names no element of W."""
+        d_gmap, d_gmap_p = _map(d_gmap, grid.num_g), _map(d_gmap_p, grid_p.num_g)
         _lib.check(_lib.lib().sgw_analytic_eval(
             self.model, self.num_g, self.z.size, self._hz, _p(self.coeff),
             _cplx(self.symmetrize(freq)), grid.n, grid_p.n, grid.num_g, grid_p.num_g,
@@ -134,7 +147,8 @@ def sigma_correlation(grid: CorrGrid, grid_p: CorrGrid, omega_cell: float, alpha
     gm = np.arange(grid.num_g, dtype=np.int32) if gmap is None else np.asarray(gmap, np.int32)
     gmp = np.arange(grid_p.num_g, dtype=np.int32) if gmap_p is None else np.asarray(gmap_p,
                                                                                       np.int32)
-    d_gm, d_gmp = torch.from_numpy(gm).to(dev), torch.from_numpy(gmp).to(dev)
+    d_gm = _map(torch.from_numpy(gm).to(dev), grid.num_g)
+    d_gmp = _map(torch.from_numpy(gmp).to(dev), grid_p.num_g)
     sigma = torch.zeros((freq_sigma.size, grid_p.num_g, grid.num_g), dtype=torch.complex128,
                         device=dev)
     nterm = freq_sigma.size * freq_green.size
