@@ -446,7 +446,7 @@ int sgw_green_assemble(int32_t nfreq, int32_t n, int32_t n_p, int32_t nrow,
  * nfreq / 3 support points and stores [positions, values, weights] in
  * thirds of nfreq / 3 slices (analytic.f90:174-193); SGW_AAA_POLE keeps the
  * poles whose residue exceeds thres as [poles, residues] in halves of
- * nfreq / 2 (pole_correction, analytic.f90:389-427).  Synchronises.  Errors
+ * nfreq / 2 (pole_correction, analytic.f90:389-427).  Both synchronise.  Errors
  * (SGW_E_STATE, the element's slices NaN): more relevant poles than
  * nfreq / 2 (the reference's errore), or an SGW_AAA_POLE element that is
  * not converged at nfreq / 2 support points (the Loewner submatrix would

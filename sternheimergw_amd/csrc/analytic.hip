@@ -118,6 +118,15 @@ constexpr double kPrTol = 1e-14;                        // eps14, the default to
 constexpr double kSqrtEps = 1.4901161193847656e-08;     // sqrt(epsilon(1.0_dp))
 constexpr double kDblEps = 2.220446049250313e-16;
 constexpr int kPrSmallMax = 35;                         // most points with G = 16
+// Open ranks are settled on the spot up to kPrHere elements or kPrHerePoints
+// points, else through a list: an open element holds up those that share its
+// wavefront, which the long Jacobi of many points makes dear; the list and the
+// second launch cost 10 to 30 us.  On the spot against the list: 1 element of
+// 20 points 26 us against 45, 40 000 of 20 points 256 against 281; 400 of 32
+// points 590 against 771, 1 600 670 against 770, 40 000 1 947 against 1 283; 1 600
+// of 36 points 1 107 against 1 057, 10 000 2 549 against 1 732.
+constexpr int64_t kPrHere = 1024;
+constexpr int kPrHerePoints = 20;
 
 // LDS per element: Taylor coefficients (2 G), b (G), tau (G), the matrix
 // (G x nmax), whose place the samples take before it and a after it (at least
@@ -339,11 +348,12 @@ template <int G> __device__ double2 pr_qlast(const double2 *A, const double2 *ta
 // [m, n, a_0..a_m, b_0..b_n, 0, ...] (the reference leaves whatever was there
 // beyond the coefficients; pade_eval_robust never reads it)
 //
-// EXACT: ranks by Jacobi.  Otherwise ranks by pr_rank_qr, and an element
-// where that leaves one open goes, untouched, to the list `open` (open[0]
-// their number), which a second launch with EXACT works off; with `open` null
-// an EXACT launch takes every element.
-template <int G, bool EXACT>
+// Ranks by pr_rank_qr and, where that leaves one open, by Jacobi on the spot
+// (kHere), or the element goes, untouched, to the list `open` (kList; open[0]
+// their number), which a second launch works off by Jacobi (kJacobi); with
+// `open` null that takes every element.
+enum { kHere, kList, kJacobi };
+template <int G, int RANK>
 __global__ __launch_bounds__(kPrBlock) void k_pade_robust_coeffs(
     int64_t ne, int N, double radius, int nmax, double2 *__restrict__ w,
     int32_t *__restrict__ open) {
@@ -357,8 +367,8 @@ __global__ __launch_bounds__(kPrBlock) void k_pade_robust_coeffs(
   __syncthreads();
   const int grp = threadIdx.x / G, l = threadIdx.x % G;
   const int64_t at = (int64_t)blockIdx.x * (blockDim.x / G) + grp;
-  if (at >= (EXACT && open ? open[0] : ne)) return;
-  const int64_t e = EXACT && open ? open[1 + at] : at;
+  if (at >= (RANK == kJacobi && open ? open[0] : ne)) return;
+  const int64_t e = RANK == kJacobi && open ? open[1 + at] : at;
   double2 *cc = pr_lds + (size_t)grp * pr_group_lds<G>(nmax);
   double2 *bv = cc + 2 * G;
   double2 *tau = bv + G;
@@ -429,11 +439,15 @@ __global__ __launch_bounds__(kPrBlock) void k_pade_robust_coeffs(
     // diagonal hopping (:318-363): while rank(C) < n, shrink m and n
     while (n > 0) {
       pr_build<G>(A, cc, m, n, l, 1.0);
-      const int rho = EXACT ? pr_rank<G>(A, n + 1, n, l, abs_tol)
-                            : pr_rank_qr<G>(A, n + 1, n, l, abs_tol);
-      if (!EXACT && rho < 0) {
+      int rho = RANK == kJacobi ? pr_rank<G>(A, n + 1, n, l, abs_tol)
+                                : pr_rank_qr<G>(A, n + 1, n, l, abs_tol);
+      if (RANK == kList && rho < 0) {
         if (l == 0) open[1 + atomicAdd(open, 1)] = (int32_t)e;
         return;
+      }
+      if (RANK == kHere && rho < 0) {
+        pr_build<G>(A, cc, m, n, l, 1.0);
+        rho = pr_rank<G>(A, n + 1, n, l, abs_tol);
       }
       if (rho == n) break;
       m -= n - rho;
@@ -506,6 +520,27 @@ __global__ __launch_bounds__(kPrBlock) void k_pade_robust_coeffs(
     w[(int64_t)s * ne + e] = v;
   }
 }
+
+// count words of device memory that are given back in the order of the stream's
+// work, without a wait; p is null where there is none
+struct StreamList {
+  StreamList(hipStream_t st, int64_t count) : st_(st) {
+    if (count > 0 && hipMallocAsync(reinterpret_cast<void **>(&p), sizeof(int32_t) * count, st) !=
+                         hipSuccess) {
+      (void)hipGetLastError();
+      p = nullptr;
+    }
+  }
+  ~StreamList() {
+    if (p) (void)hipFreeAsync(p, st_);
+  }
+  StreamList(const StreamList &) = delete;
+  StreamList &operator=(const StreamList &) = delete;
+  int32_t *p = nullptr;
+
+ private:
+  hipStream_t st_;
+};
 
 // analytic_eval (analytic.f90:276-345): out(r, c) for r < num_g, c < num_g_p
 // from the coefficients of element (gmap[r], gmap_p[c]); out zeroed before
@@ -719,40 +754,43 @@ extern "C" int sgw_analytic_coeff(int32_t model, double thres, int32_t num_g, in
                     "pade_coeff_robust: frequencies must span circle in the complex plane");
       SGW_REQUIRE(radius > 0.0, SGW_E_ARG, "pade_robust: radius in the complex plane must be > 0");
       const int nmax = nfreq / 2 - 2;
-      DevBuf<int32_t> open;
-      auto go = [&](auto group) {
-        constexpr int G = decltype(group)::value;
-        const int bytes = (int)sizeof(double2) * pr_group_lds<G>(nmax);   // <= 18432
-        const int per = std::min(kPrBlock / G, kPrLdsMax / bytes);
-        const unsigned grid = (unsigned)((ne + per - 1) / per);
-        if (!open.p) {
-          k_pade_robust_coeffs<G, true><<<grid, G * per, (size_t)per * bytes, st>>>(
-              ne, nfreq, radius, nmax, w, nullptr);
-          return;
-        }
-        k_pade_robust_coeffs<G, false><<<grid, G * per, (size_t)per * bytes, st>>>(
-            ne, nfreq, radius, nmax, w, open.p);
-        // as many groups as elements might be open: those past the list's end leave at once
-        k_pade_robust_coeffs<G, true><<<grid, G * per, (size_t)per * bytes, st>>>(
-            ne, nfreq, radius, nmax, w, open.p);
-      };
-      // the list of open elements; a stream under capture takes every element
-      // through Jacobi instead (no allocation there)
+      // The list of open elements belongs to the stream and is given back in its
+      // order, so that the call returns behind its launches.  A stream under
+      // capture takes every element through Jacobi; without memory for the list
+      // open ranks are settled on the spot.
       hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
       if (hipStreamIsCapturing(st, &cap) != hipSuccess) {
         (void)hipGetLastError();
         cap = hipStreamCaptureStatusActive;
       }
-      if (cap == hipStreamCaptureStatusNone && ne < (1ll << 31) - 1) {
-        open.alloc((size_t)ne + 1);
-        SGW_HIP(hipMemsetAsync(open.p, 0, sizeof(int32_t), st));
-      }
+      const bool capture = cap != hipStreamCaptureStatusNone;
+      const bool here = ne <= kPrHere || nfreq <= kPrHerePoints || ne >= (1ll << 31) - 1;
+      StreamList open(st, capture || here ? 0 : ne + 1);
+      auto go = [&](auto group) {
+        constexpr int G = decltype(group)::value;
+        const int bytes = (int)sizeof(double2) * pr_group_lds<G>(nmax);   // <= 18432
+        const int per = std::min(kPrBlock / G, kPrLdsMax / bytes);
+        const unsigned grid = (unsigned)((ne + per - 1) / per);
+        auto launch = [&](auto rank) {
+          k_pade_robust_coeffs<G, decltype(rank)::value>
+              <<<grid, G * per, (size_t)per * bytes, st>>>(ne, nfreq, radius, nmax, w, open.p);
+          SGW_HIP(hipGetLastError());
+        };
+        using std::integral_constant;
+        if (open.p) {
+          SGW_HIP(hipMemsetAsync(open.p, 0, sizeof(int32_t), st));
+          launch(integral_constant<int, kList>{});
+          // as many groups as elements might be open: those past the list's end
+          // leave at once
+          launch(integral_constant<int, kJacobi>{});
+        } else if (capture) {
+          launch(integral_constant<int, kJacobi>{});
+        } else {
+          launch(integral_constant<int, kHere>{});
+        }
+      };
       if (nfreq <= kPrSmallMax) go(std::integral_constant<int, 16>{});
       else go(std::integral_constant<int, 32>{});
-      if (open.p) {
-        SGW_HIP(hipGetLastError());
-        SGW_HIP(hipStreamSynchronize(st));  // the list is freed here
-      }
     } else if (model == SGW_AAA_APPROX || model == SGW_AAA_POLE) {
       // aaa_generate per element on the symmetrised mesh (analytic.f90:162-199)
       const Mesh m = make_mesh(nfreq, h_z, h_src);
