@@ -559,10 +559,11 @@ int sgw_kernel_timing_query(const char *name, double *total_ms, int64_t *launche
 /* Launch-shape autotuning.  No counterpart in the reference.  The split plane
  * transforms of cubic boxes up to 48 (three planes on two wavefronts, one
  * plane per wavefront, one plane on two, two planes on two) and the final assembly of
- * an application (16, 32 or 64 plane waves per block) have several launch
+ * an application (64, 32 or 16 plane waves per block) have several launch
  * shapes with the same results; the first application of each size class (batch size
  * rounded up to a power of two) times every shape once and keeps the fastest.
- * SGW_AUTOTUNE=0 in the environment keeps the first shape.  Returns the
+ * SGW_AUTOTUNE=0 in the environment keeps the default: the first plane shape
+ * that fits, the widest assembly block that fills the chip.  Returns the
  * candidate index chosen for `key` ("plane<box>/M<m>/b<band>/n<class>",
  * "assemble/n<class>/g<groups>/p<projectors>"), -1 if none yet. */
 int sgw_autotune_choice(const char *key);

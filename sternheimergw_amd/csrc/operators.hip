@@ -1982,7 +1982,7 @@ void PwOperator::apply_work(hipStream_t st, int nvec, const double2 *in, int64_t
     // 64 plane waves x 4 vector groups, 32 x 8 or 16 x 16 to a block.  Wide
     // blocks read a projector value once for four vectors; narrow ones fill the
     // chip for a small batch and have fewer products in a row.  The widest with
-    // kAsmBlocks blocks goes first: 48^3 (48 projectors, 26 chunks of 64) 512
+    // kAsmBlocks blocks is the default: 48^3 (48 projectors, 26 chunks of 64) 512
     // vectors 21.0 / 23.9 / 28.8 us, 256 vectors 16.0 / 15.2 / 17.7, 64 vectors
     // 14.4 / 10.9 / 9.6 (8.7 with 16 values together), 16 vectors 12.6 / 9.1 / 7.8;
     // 36^3 (26 projectors, 10 chunks) 512 vectors 12.6 / 10.8 / 11.2, 256 vectors
@@ -2005,12 +2005,14 @@ void PwOperator::apply_work(hipStream_t st, int nvec, const double2 *in, int64_t
                           in + (int64_t)(nvec - 1) * in_stride + ld <= out;
     const std::string key = "assemble/n" + std::to_string(size_class(nvec)) + "/g" +
                             std::to_string(ngroup_) + "/p" + std::to_string(nproj_);
-    autotune(key, disjoint ? 3 : 1, st, [&](int c) {
-      const int shape = (first + c) % 3;
-      if (shape == 0) launch_asm(std::integral_constant<int, 64>{});
-      else if (shape == 1) launch_asm(std::integral_constant<int, 32>{});
-      else launch_asm(std::integral_constant<int, 16>{});
-    });
+    autotune(
+        key, disjoint ? 3 : 1, st,
+        [&](int c) {
+          if (c == 0) launch_asm(std::integral_constant<int, 64>{});
+          else if (c == 1) launch_asm(std::integral_constant<int, 32>{});
+          else launch_asm(std::integral_constant<int, 16>{});
+        },
+        first);
   }
   SGW_HIP(hipGetLastError());
 }

@@ -32,7 +32,7 @@ int autotune_choice(const std::string &key) {
 }
 
 int autotune(const std::string &key, int ncand, hipStream_t st,
-             const std::function<void(int)> &launch) {
+             const std::function<void(int)> &launch, int def) {
   const int forced = forced_candidate();
   if (forced >= 0) {
     const int c = forced < ncand ? forced : ncand - 1;
@@ -40,8 +40,8 @@ int autotune(const std::string &key, int ncand, hipStream_t st,
     return c;
   }
   if (ncand <= 1 || !tuning_enabled()) {
-    launch(0);
-    return 0;
+    launch(def);
+    return def;
   }
   {
     std::lock_guard<std::mutex> lk(g_tune_mu);
@@ -54,18 +54,19 @@ int autotune(const std::string &key, int ncand, hipStream_t st,
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
   SGW_HIP(hipStreamIsCapturing(st, &cap));
   if (cap != hipStreamCaptureStatusNone) {
-    launch(0);
-    return 0;
+    launch(def);
+    return def;
   }
   // each candidate three times: the first launch also loads the kernel's
   // code and is not timed; the faster of the other two counts
   hipEvent_t e0, e1;
   SGW_HIP(hipEventCreate(&e0));
   SGW_HIP(hipEventCreate(&e1));
-  int best = 0;
+  int best = def;
   float best_ms = 0.f;
   try {
-    for (int i = 0; i < ncand; ++i) {
+    for (int k = 0; k < ncand; ++k) {
+      const int i = (def + k) % ncand;
       launch(i);
       float fastest = 0.f;
       for (int rep = 0; rep < 2; ++rep) {
@@ -77,7 +78,7 @@ int autotune(const std::string &key, int ncand, hipStream_t st,
         SGW_HIP(hipEventElapsedTime(&ms, e0, e1));
         if (rep == 0 || ms < fastest) fastest = ms;
       }
-      if (i == 0 || fastest < best_ms) {
+      if (k == 0 || fastest < best_ms) {
         best = i;
         best_ms = fastest;
       }
