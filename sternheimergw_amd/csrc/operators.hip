@@ -1665,8 +1665,15 @@ PwOperator::PwOperator(const PwDesc &desc) {
   // 39.8 against 33.4 (20 Ha); the 32^3 box 41 to 46 against 34, the 36^3 box
   // 66 to 86 against 38.  The number of vectors has no part in the rule, so that
   // a vector's result does not depend on its batch.
+  // A block reads the projectors for its vector alone, the batched kernels
+  // once for 16: with more than 24 K values of them (plane waves x projectors) a
+  // large batch is the slower for it.  1024 vectors, an application against
+  // batched: 9 K values 94 us against 99, 19 K 115 and 114, 21 K 113 and 112; 38 K
+  // 157 against 134, 45 K 144 against 131, 90 K 212 against 178 (1 vector: 56
+  // against 50).
+  constexpr int64_t kBlockProj = 24 * 1024;
   block_ = n1_ == 24 && n2_ == 24 && n3_ == 24 && columns_contiguous_ && fuse_stages_ &&
-           split_planes_ && band_planes_ &&
+           split_planes_ && band_planes_ && nproj_ * ld <= kBlockProj &&
            pwblock::layout(n1_, nc1_, ncs_, ld, nproj_).total * sizeof(double2) <= pwblock::kLds;
   SGW_HIP(hipDeviceSynchronize());
 }

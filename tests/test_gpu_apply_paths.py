@@ -169,3 +169,27 @@ def test_gradient_boxes(n, nq, nshift):
     Lo, go = ao.l_and_grad(w, list(range(w.nsys)), -w.rhs, weight, threshold=1e-13)
     assert abs(L - Lo) <= 1e-10 * abs(Lo)
     assert np.abs(grad.cpu().numpy() - go).max() <= 1e-9 * np.abs(go).max()
+
+
+def _block_launches(op, ld, npw, nv):
+    rng = np.random.Generator(np.random.PCG64(nv))
+    x = np.zeros((nv, ld), dtype=np.complex128)
+    x[:, :npw] = rng.standard_normal((nv, npw)) + 1j * rng.standard_normal((nv, npw))
+    L, ms, count = _lib.lib(), ctypes.c_double(), ctypes.c_int64()
+    _lib.check(L.sgw_kernel_timing(2))
+    op.apply(x, np.full(nv, 0.3 + 0.1j), group=np.zeros(nv, np.int32))
+    _lib.check(L.sgw_kernel_timing_query(b"pw_block", ctypes.byref(ms), ctypes.byref(count)))
+    _lib.check(L.sgw_kernel_timing(0))
+    return count.value
+
+
+@pytest.mark.parametrize("ecut,nbeta,block", [(6.0, 0, 1), (6.0, 128, 1), (6.0, 129, 0),
+                                               (10.0, 48, 1), (10.0, 60, 0), (12.0, 4, 0)])
+def test_one_block_needs_few_projectors(ecut, nbeta, block):
+    """24^3: one block per vector up to 24 K projector values (192 places for the
+    plane waves at 6 Ha, 448 at 10 Ha) and some 11 Ha, for any batch."""
+    print(f"one block per vector {ecut} Ha, {nbeta} projectors", flush=True)
+    w, op = _cell(24, ecut, nbeta, 0, 1)
+    assert nbeta * w.ld <= 24 * 1024 or block == 0
+    for nv in (1, 300):
+        assert _block_launches(op, w.ld, w.npw[0], nv) == block
