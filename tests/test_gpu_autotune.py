@@ -1,6 +1,7 @@
-"""The autotuner's candidates of the assembly are shapes: candidate 0, 1 and 2
-are 64, 32 and 16 plane waves to a block, whatever the batch or the sphere, so
-that a choice that was timed is the one that runs wherever its key is met."""
+"""The autotuner's candidates are shapes with the same results, and their numbers
+are absolute: candidate 0, 1 and 2 of the assembly are 64, 32 and 16 plane waves
+to a block, whatever the batch or the sphere, so that a choice that was timed
+is the one that runs wherever its key is met."""
 import re
 
 import numpy as np
@@ -8,6 +9,7 @@ import pytest
 import torch
 from test_gpu_apply_paths import _cell
 
+from oracle import oracle as orc
 from sternheimergw_amd import _lib
 
 pytestmark = pytest.mark.gpu
@@ -51,3 +53,39 @@ def test_choice_holds_for_its_key(monkeypatch):
         assert _assembly_widths(op, w.ld, nv) == [WIDTH[choice]]
     w2, op2 = _cell(36, 9.0, 9, 4, 1)         # another sphere, the same key
     assert _assembly_widths(op2, w2.ld, 200) == [WIDTH[choice]]
+
+
+@pytest.mark.parametrize("n,ecut,ngroup", [(24, 12.0, 3), (24, 20.0, 2), (32, 9.0, 3)])
+def test_batched_shapes_agree_bitwise(n, ecut, ngroup, monkeypatch):
+    """Ragged k+q groups on boxes whose vectors the batched kernels take: every
+    launch shape of the plane transforms (three planes on two wavefronts, one on
+    one, one on two, two on two) and of the assembly gives the same bits, and
+    the tuned run records its choices, so that the shapes did run."""
+    print(f"batched shapes {n}^3 {ecut} Ha", flush=True)
+    monkeypatch.delenv("SGW_AUTOTUNE", raising=False)
+    w, op = _cell(n, ecut, 8, 5, ngroup)
+    rng = np.random.Generator(np.random.PCG64(21))
+    nv = 13
+    grp = (np.arange(nv) % ngroup).astype(np.int32)
+    x = np.zeros((nv, w.ld), dtype=np.complex128)
+    for v in range(nv):
+        m = w.npw[grp[v]]
+        x[v, :m] = rng.standard_normal(m) + 1j * rng.standard_normal(m)
+    sig = rng.standard_normal(nv) + 1j * rng.standard_normal(nv)
+    out = []
+    for c in range(4):
+        monkeypatch.setenv("SGW_AUTOTUNE_FORCE", str(c))
+        out.append(op.apply(x, sig, group=grp))
+    monkeypatch.delenv("SGW_AUTOTUNE_FORCE")
+    tuned = op.apply(x, sig, group=grp)
+    for o in out[1:] + [tuned]:
+        assert np.array_equal(o, out[0])
+    half = int(max(np.abs(s.mill).max() for s in w.spheres))
+    band = half if 4 <= half <= {24: 5, 32: 7}[n] else -1
+    choice = _lib.lib().sgw_autotune_choice
+    assert choice(f"plane{n}/M{half}/b{band}/n16".encode()) >= 0
+    assert choice(f"assemble/n16/g{ngroup}/p13".encode()) >= 0
+    for v in range(ngroup):
+        m = w.npw[grp[v]]
+        ref = orc.PwOp(w, int(grp[v])).apply(x[v, :m], sig[v])
+        assert np.linalg.norm(out[0][v, :m] - ref) <= 1e-12 * np.linalg.norm(ref)
