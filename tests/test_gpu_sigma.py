@@ -150,3 +150,34 @@ def test_conv_tiles(n, nout, nin):
     got = _from_dev_colmajor(d_s, n)
     for i in range(nout):
         assert np.linalg.norm(got[i] - ref[i]) <= FP64_TOL * np.linalg.norm(ref[i]), i
+
+
+@pytest.mark.parametrize("n,nout,nin,tile", [
+    (449, 3, 1, "_small"), (1025, 1, 1, "_small"),                     # 16 x 16, K split
+    (481, 3, 2, "<1, 1>"), (593, 2, 1, "<1, 1>"), (849, 1, 2, "<1, 1>"),  # 32 x 32
+    (673, 2, 2, "<2, 1>"), (945, 1, 1, "<2, 1>"),                      # 64 x 32
+    (641, 4, 1, "<2, 2>"), (737, 3, 1, "<2, 2>")])                     # 64 x 64
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_conv_each_tile(n, nout, nin, tile, accumulate):
+    """Every tile of the FP64 kernel at sizes one or a half tile past its multiples,
+    padded rows, with and without a Sigma to add to; the kernel's name says
+    that it is the tile meant."""
+    print(f"sigma_conv tile {tile} n={n} nout={nout} nin={nin} acc={accumulate}", flush=True)
+    rng = np.random.Generator(np.random.PCG64(n))
+    ld = n + 3
+    G, W, S0 = _rand(rng, nout, nin, n, n), _rand(rng, nin, n, n), _rand(rng, nout, n, n)
+    wt = rng.uniform(0.1, 1.0, nin)
+    alpha = complex(0.7, -0.2)
+    ref = S0 if accumulate else np.zeros_like(S0)
+    ref = ref + alpha * sum(wt[j] * np.matmul(G[:, j], W[j]) for j in range(nin))
+    d_g, d_w, d_s = (_to_dev_colmajor(m, ld) for m in (G, W, S0))
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as prof:
+        sigma.conv_device(d_g, d_w, torch.from_numpy(wt).to(DEV), d_s, n, ld, nout, nin, alpha,
+                          accumulate=accumulate)
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events() if "k_sigma_f64" in e.name]
+    assert len(names) == 1 and "k_sigma_f64" + tile in names[0], names
+    got = _from_dev_colmajor(d_s, n)
+    for i in range(nout):
+        assert np.linalg.norm(got[i] - ref[i]) <= FP64_TOL * np.linalg.norm(ref[i]), i
+    assert not d_s.cpu().numpy()[..., n:].any()
