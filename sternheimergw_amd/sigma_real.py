@@ -127,8 +127,9 @@ def _green_offsets(d_green_r, num_green, size):
     if d_green_r.shape[0] < num_green:
         raise IndexError(f"{num_green} Green's functions needed, the stack holds "
                          f"{d_green_r.shape[0]}")
-    one = d_green_r[0]
-    if one.dtype != torch.complex128 or one.numel() < size or not one.is_contiguous():
+    one = d_green_r if d_green_r.is_contiguous() else d_green_r[0]
+    held = d_green_r.numel() // d_green_r.shape[0] if one.is_contiguous() else 0
+    if d_green_r.dtype != torch.complex128 or held < size:
         raise ValueError("each G(r, r') must be a contiguous complex128 (nr_p, nr) matrix")
     return np.arange(num_green, dtype=np.int64) * d_green_r.stride(0)
 
@@ -147,8 +148,9 @@ def sigma_correlation(grid: CorrGrid, grid_p: CorrGrid, omega_cell: float, alpha
     gm = np.arange(grid.num_g, dtype=np.int32) if gmap is None else np.asarray(gmap, np.int32)
     gmp = np.arange(grid_p.num_g, dtype=np.int32) if gmap_p is None else np.asarray(gmap_p,
                                                                                       np.int32)
-    d_gm = _map(torch.from_numpy(gm).to(dev), grid.num_g)
-    d_gmp = _map(torch.from_numpy(gmp).to(dev), grid_p.num_g)
+    gm, gmp = (m if m.size >= num else np.pad(m.ravel(), (0, num - m.size), constant_values=-1)
+               for m, num in ((gm, grid.num_g), (gmp, grid_p.num_g)))     # as _map
+    d_gm, d_gmp = torch.from_numpy(gm).to(dev), torch.from_numpy(gmp).to(dev)
     sigma = torch.zeros((freq_sigma.size, grid_p.num_g, grid.num_g), dtype=torch.complex128,
                         device=dev)
     nterm = freq_sigma.size * freq_green.size
