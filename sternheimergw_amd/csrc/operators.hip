@@ -2089,7 +2089,8 @@ void PwOperator::grad_accumulate(hipStream_t st, int np, const double2 *x, const
               "pw operator: the V_loc gradient needs a cubic 24/32/36/48 box");
   SGW_REQUIRE(sizeof(double2) * (nslot_ + (size_t)nc1_ * n1_ + (size_t)n1_ * n1_) <= 64 * 1024,
               SGW_E_ARG, "pw operator: gradient plane does not fit in LDS");
-  // at most 40 KB by the line above
+  // the limit is that of a plane kept in LDS beside its rows; the kernel keeps
+  // rows only, 18 to 55 KB at the largest spheres within it
   const size_t lds = sizeof(double2) * 2 * (size_t)nc1_ * (n1_ + 1);
   SGW_REQUIRE(nb >= 1 && nb < 65536, SGW_E_ARG, "pw operator: bad gradient partial count");
   ensure_scratch(np);

@@ -7,7 +7,7 @@ same sum over frequencies is sigma.py.
 
 Device tensors use the layout [f][c][r] of Fortran arrays (r, c, f); the
 arithmetic is the library's (sgw_analytic_coeff, sgw_analytic_eval,
-sgw_sigma_prod)."""
+sgw_sigma_prod, sgw_sigma_correlation)."""
 from __future__ import annotations
 
 import ctypes
